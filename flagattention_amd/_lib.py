@@ -86,3 +86,23 @@ def get():
                 "`make -C flagattention_amd/csrc` -- there is no fallback implementation")
         _lib = bind(LIB_PATH)
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The native host path of the operators for GPU tensors (``_host.so``, built with the kernel library from
+    ``csrc/host.cpp``); raises if it is not there."""
+    global _native
+    if _native is None:
+        get()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError("_host.so is not built for this interpreter and torch; build it with "
+                               "`make -C flagattention_amd/csrc` -- there is no fallback implementation") from e
+        from . import _abi, flash, piecewise
+        _host.bind(_abi.check, flash.backward_settings, piecewise.backward_settings)
+        _native = _host
+    return _native

@@ -1,0 +1,617 @@
+// Host path of the operators for GPU tensors: argument checks, launch decisions, allocations and launches of one
+// call in one native function, with native autograd nodes for the two operators that have gradients.
+//
+// Why it is native: the kernels of a short call take 10-40 us, and the same work done in Python through ctypes took
+// longer than they do -- 38 us for a decode step, 20 us for a paged one, 195 us for a forward and backward over
+// 512 tokens (of 42 us of kernels).
+//
+// The Python modules hold the reference form of every decision made here (`flash.py`, `split_kv.py`, `paged.py`,
+// `piecewise.py`).  It runs whenever a tile-config hook has been replaced, for tensors that are not on a GPU, and
+// for every call this file does not take (it then answers NotImplemented, before any effect); arguments that are
+// in error are among those, so that their messages have one source.  `decisions()` exposes the numbers chosen here
+// to the test that compares them with the Python functions.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <algorithm>
+#include <cmath>
+
+#include "../../include/flagattn.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// Python callables bound once at import: abi.check (raises for an error code), the per-backward settings.
+PyObject* g_check = nullptr;
+PyObject* g_flash_settings = nullptr;
+PyObject* g_piecewise_settings = nullptr;
+
+// Thrown through code that does not hold the GIL; the Python error travels with it.
+[[noreturn]] void throw_python_error() {
+  python_error e;
+  e.persist();
+  throw std::move(e);
+}
+
+void check(int code, const char* what) {
+  if (code == 0) return;
+  pybind11::gil_scoped_acquire gil;
+  PyObject* r = PyObject_CallFunction(g_check, "is", code, what);
+  if (!r) throw_python_error();
+  Py_DECREF(r);
+  throw std::runtime_error(std::string(what) + ": the kernel library failed");
+}
+
+// ---------------------------------------------------------------------------------------------- decisions ----
+int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+constexpr int kSplitBlockM = 16, kSplitBlockN = 128;   // split_kv.SPLIT_BLOCK_M, SPLIT_BLOCK_N
+constexpr int kDecodeMaxRows = 16;                     // split_kv.DECODE_MAX_ROWS
+
+// split_kv.num_splits_heuristic
+int num_splits_heuristic(int64_t B, int64_t H, int64_t M, int64_t N, int cus, int max_splits) {
+  const int64_t base = B * H * cdiv(M, kSplitBlockM);
+  if ((double)base >= 0.8 * cus) return 1;
+  const int64_t units = cdiv(N, kSplitBlockN), limit = std::min<int64_t>({cus, units, max_splits});
+  auto efficiency = [&](int64_t s) {
+    const double waves = (double)(base * s) / cus;
+    return waves / std::ceil(waves);
+  };
+  auto last_is_empty = [&](int64_t s) { const int64_t per = cdiv(units, s); return s > 1 && per * s - units >= per; };
+  double best = 0.0;
+  for (int64_t s = 1; s <= limit; ++s)
+    if (!last_is_empty(s)) best = std::max(best, efficiency(s));
+  for (int64_t s = 1; s <= limit; ++s)
+    if (!last_is_empty(s) && efficiency(s) >= 0.85 * best) return (int)s;
+  return 1;
+}
+
+// split_kv.choose_num_splits
+int choose_num_splits(int64_t B, int64_t H, int64_t Hk, int64_t M, int64_t N, int cus) {
+  const int64_t base = B * Hk * cdiv(H / Hk * M, 16), units = cdiv(N, kSplitBlockN);
+  const int64_t want = cdiv(2 * (int64_t)cus, base), cap = std::max<int64_t>(1, N / 512);
+  int64_t splits = std::min(std::max<int64_t>(1, std::min<int64_t>({want, cap, 128})), units);
+  while (splits > 1 && cdiv(units, splits) * (splits - 1) >= units) --splits;
+  return (int)splits;
+}
+
+// split_kv._split_size
+int split_size(int64_t N, int splits) { return (int)(cdiv(cdiv(N, kSplitBlockN), splits) * kSplitBlockN); }
+
+// flash.wide_key_splits
+int wide_key_splits(int64_t B, int64_t H, int64_t M, int64_t N, int64_t D, int cus) {
+  if (D != 128 || M < 256) return 1;
+  const int64_t wgs = cdiv(M, 256) * H * B, pieces = std::min<int64_t>(cus / wgs, N / 1024);
+  return pieces < 2 || 4 * pieces * wgs < 3 * (int64_t)cus ? 1 : (int)pieces;
+}
+
+// flash.dkdv_heads_per_slice
+int dkdv_heads_per_slice(int64_t B, int64_t H, int group, int64_t N, int cus) {
+  const int64_t blocks = cdiv(N, 128);
+  for (int chunk = group; chunk > 0; --chunk)
+    if (group % chunk == 0 && blocks * B * (H / chunk) >= 2 * (int64_t)cus) return chunk;
+  return 1;
+}
+
+// flash.ds_heads_per_launch
+int64_t ds_heads_per_launch(int64_t B, int64_t H, int group, int64_t M, int64_t N, int64_t D, int64_t limit_mib, int grids) {
+  if (D < 128 || M * N < 1024 * 1024 || limit_mib <= 0) return 0;
+  const int64_t per_head = (int64_t)grids * fa_bwd_ds_workspace_mib(1, 1, (int)M, (int)N);
+  const int64_t fit = limit_mib / per_head;
+  return fit >= B * H ? B * H : fit / group * group;
+}
+
+// paged.choose_launch: workgroups of the balanced launch, 0 = one workgroup per (sequence, kv head) pair
+int balanced_workgroups(int64_t seqs, int64_t Hkv, int64_t group, int64_t D, int64_t max_context, int cus) {
+  const int wgs = cus * (D <= 128 ? 2 : 1);
+  return seqs * Hkv * cdiv(group, 16) >= 8 * (int64_t)wgs && max_context <= 2048 ? 0 : wgs;
+}
+
+// ------------------------------------------------------------------------------------------------ tensors ----
+int dtype_code(const Tensor& t) { return t.scalar_type() == at::kHalf ? FA_F16 : FA_BF16; }
+
+// _abi.is_kernel_ready
+bool is_kernel_ready(const Tensor& t) {
+  const auto sizes = t.sizes(), strides = t.strides();
+  const int64_t last = t.dim() - 1;
+  if (strides[last] != 1 || ((uintptr_t)t.const_data_ptr() & 15)) return false;
+  for (int64_t i = 0; i < last; ++i)
+    if (sizes[i] > 1 && strides[i] % 8) return false;
+  return true;
+}
+Tensor kernel_ready(const Tensor& t) { return is_kernel_ready(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+
+fa_view4 view4(const Tensor& t) {
+  const auto n = t.sizes(), s = t.strides();
+  // the stride of a dimension of extent 1 is never used; torch leaves arbitrary values there
+  return fa_view4{const_cast<void*>(t.const_data_ptr()), n[0] > 1 ? s[0] : 0, n[1] > 1 ? s[1] : 0, n[2] > 1 ? s[2] : 0};
+}
+// heads [h0, h1) of batch entry b
+fa_view4 slice4(const Tensor& t, int64_t b, int64_t h0) {
+  fa_view4 v = view4(t);
+  v.ptr = (char*)v.ptr + (b * v.stride_b + h0 * v.stride_h) * (int64_t)t.element_size();
+  return v;
+}
+
+Tensor empty(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) {
+  return at::detail::empty_cuda(shape, type, like.device(), std::nullopt);
+}
+// torch.empty_like(t) where the kernels can write that layout, otherwise contiguous
+Tensor empty_result(const Tensor& t) {
+  if (t.is_contiguous()) return empty(t.sizes(), t.scalar_type(), t);
+  Tensor o = at::empty_like(t);
+  return is_kernel_ready(o) ? o : empty(t.sizes(), t.scalar_type(), t);
+}
+
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+float* f32(const Tensor& t) { return (float*)const_cast<void*>(t.const_data_ptr()); }
+
+bool is_operand(const Tensor& t, const Tensor& first) {
+  return t.is_cuda() && t.dim() == 4 && t.layout() == at::kStrided && t.device() == first.device() &&
+         t.scalar_type() == first.scalar_type();
+}
+bool type_ok(const Tensor& t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
+bool fits_int(std::initializer_list<int64_t> xs) {
+  for (int64_t x : xs)
+    if (x <= 0 || x > 0x7fffffff) return false;
+  return true;
+}
+
+// dS of `heads` heads, or an undefined tensor when the allocator has no memory left (the caller then recomputes)
+Tensor ds_workspace(const Tensor& like, int64_t B, int64_t H, int64_t M, int64_t N, int grids) {
+  const int mib = fa_bwd_ds_workspace_mib((int)B, (int)H, (int)M, (int)N);
+  if (mib <= 0) check(mib ? mib : FA_ERR_BAD_ARGUMENT, "fa_bwd_ds_workspace_mib");
+  try {
+    return empty({(int64_t)grids * ((int64_t)mib << 20)}, at::kByte, like);
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
+}
+
+// The settings a backward reads when it runs: calls the (replaceable) tile hook, returns the dS workspace limit.
+int64_t backward_settings(PyObject* callable, int64_t B, int64_t H, int64_t M, int64_t N, int64_t D, bool causal) {
+  pybind11::gil_scoped_acquire gil;
+  PyObject* r = PyObject_CallFunction(callable, "LLLLLO", (long long)B, (long long)H, (long long)M, (long long)N,
+                                      (long long)D, causal ? Py_True : Py_False);
+  if (!r) throw_python_error();
+  const int64_t limit = PyLong_AsLongLong(r);
+  Py_DECREF(r);
+  if (limit == -1 && PyErr_Occurred()) throw_python_error();
+  return limit;
+}
+
+// ------------------------------------------------------------------------------------------ flash attention ----
+struct FlashCall {
+  bool causal, want_total;
+  double scale, dropout_p;
+  uint64_t seed, offset;
+};
+
+// pieces > 0: the split kernel over that many pieces of the key axis and the merge; 0: the dense kernel
+struct FlashPlan { int pieces; };
+
+// false: the combination is an error (dropout on a split shape)
+bool plan_flash(FlashPlan& plan, int64_t B, int64_t H, int64_t Hk, int64_t M, int64_t N, int64_t D, bool dropout,
+                double scale, int64_t row_bytes, int cus) {
+  const int splits = num_splits_heuristic(B, H, M, N, cus, 128);
+  plan.pieces = 0;
+  if (splits > 1 && dropout) return false;
+  if (splits > 1 || (M <= kDecodeMaxRows && N >= 1024 && !dropout)) {
+    plan.pieces = choose_num_splits(B, H, Hk, M, N, cus);
+  } else if (!dropout && scale > 0 && row_bytes < (1 << 24)) {
+    const int pieces = wide_key_splits(B, H, M, N, D, cus);
+    if (pieces > 1) plan.pieces = pieces;
+  }
+  return true;
+}
+
+// o, L and (if asked for) the column sums
+variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, const FlashCall& c, const FlashPlan& plan) {
+  const int B = (int)q.size(0), H = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3);
+  const int Hk = (int)k.size(1), N = (int)k.size(2), type = dtype_code(q);
+  void* stream = stream_of(q);
+  const fa_view4 vq = view4(q), vk = view4(k), vv = view4(v);
+  Tensor o, L;
+  if (plan.pieces > 0) {
+    const int S = plan.pieces;
+    Tensor part_lse = empty({B, H, S, M}, at::kFloat, q), part_o = empty({B, H, S, M, D}, at::kHalf, q);
+    check(fa_splitkv_fwd(type, &vq, &vk, &vv, part_o.mutable_data_ptr(), f32(part_lse), B, H, Hk, M, N, D, c.causal,
+                         (float)c.scale, S, split_size(N, S), stream), "fa_splitkv_fwd");
+    if (S == 1) {   // nothing to merge: the single piece is the result (a cast at most)
+      o = part_o.squeeze(2).to(q.scalar_type());
+      L = part_lse.squeeze(2);
+    } else {
+      L = empty({B, H, M}, at::kFloat, q);
+      o = empty_result(q);
+      const fa_view4 vo = view4(o);
+      check(fa_splitkv_combine(type, part_o.const_data_ptr(), f32(part_lse), &vo, f32(L), B, H, M, D, S, stream),
+            "fa_splitkv_combine");
+    }
+  } else {
+    o = empty_result(q);
+    L = empty({B, H, M}, at::kFloat, q);
+    const fa_view4 vo = view4(o);
+    check(fa_fwd(type, &vq, &vk, &vv, &vo, f32(L), B, H, Hk, M, N, D, c.causal, (float)c.scale, (float)c.dropout_p,
+                 c.seed, c.offset, 0, stream), "fa_fwd");
+  }
+  variable_list out = {o, L};
+  if (c.want_total) {
+    Tensor tot = empty({B, H, N}, at::kFloat, q);
+    check(fa_total_attn(type, &vq, &vk, f32(L), f32(tot), B, H, Hk, M, N, D, c.causal, (float)c.scale, stream),
+          "fa_total_attn");
+    out.push_back(tot);
+  }
+  return out;
+}
+
+variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& L,
+                             const Tensor& grad, const FlashCall& c, int64_t limit_mib) {
+  const int B = (int)q.size(0), H = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3);
+  const int Hk = (int)k.size(1), N = (int)k.size(2), group = H / Hk, type = dtype_code(q);
+  const Tensor g = kernel_ready(grad);
+  void* stream = stream_of(q);
+  const fa_view4 vq = view4(q), vk = view4(k), vv = view4(v), vo = view4(o), vg = view4(g);
+  const float scale = (float)c.scale, p = (float)c.dropout_p;
+  Tensor delta = empty(L.sizes(), at::kFloat, q);
+  check(fa_bwd_delta(type, &vo, &vg, f32(delta), B, H, M, D, stream), "fa_bwd_delta");
+  // one slice of dK / dV per `chunk` query heads; the kernels that sum query heads are built without dropout
+  const int chunk = c.dropout_p > 0 ? 1 : dkdv_heads_per_slice(B, H, group, N, fa_num_cus());
+  const int slices = H / chunk;
+  Tensor dk = empty({B, slices, N, D}, k.scalar_type(), q), dv = empty({B, slices, N, D}, k.scalar_type(), q);
+  Tensor dq = empty({B, H, M, D}, q.scalar_type(), q);
+  const fa_view4 vdk = view4(dk), vdv = view4(dv), vdq = view4(dq);
+  int64_t heads = ds_heads_per_launch(B, H, group, M, N, D, limit_mib, 1);
+  Tensor ds;
+  if (heads >= (int64_t)B * H) ds = ds_workspace(q, B, H, M, N, 1);
+  else if (heads > 0) ds = ds_workspace(q, 1, heads = std::min<int64_t>(heads, H), M, N, 1);
+  if (!ds.defined()) {   // dS not worth keeping for this shape, or no memory for it: recompute it
+    check(fa_bwd_dkdv(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, B, H, Hk, M, N, D, c.causal,
+                      scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv");
+    check(fa_bwd_dq(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdq, B, H, Hk, M, N, D, c.causal, scale, p, c.seed,
+                    c.offset, stream), "fa_bwd_dq");
+  } else if (heads >= (int64_t)B * H) {
+    check(fa_bwd_dkdv_ds(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, ds.mutable_data_ptr(),
+                         ds.numel(), B, H, Hk, M, N, D, c.causal, scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv_ds");
+    check(fa_bwd_dq_from_ds(type, &vk, ds.const_data_ptr(), ds.numel(), &vdq, B, H, Hk, M, N, D, c.causal, scale,
+                            stream), "fa_bwd_dq_from_ds");
+  } else {
+    // bounded workspace: one batch entry and `heads` query heads (whole groups) at a time; the dropout counter of a
+    // slice starts where the slice starts in the (B, H, M, N) score tensor
+    for (int64_t b = 0; b < B; ++b)
+      for (int64_t h0 = 0; h0 < H; h0 += heads) {
+        const int n = (int)(std::min<int64_t>(H, h0 + heads) - h0), kn = n / group;
+        const fa_view4 sq = slice4(q, b, h0), sk = slice4(k, b, h0 / group), sv = slice4(v, b, h0 / group),
+                       sg = slice4(g, b, h0), sdk = slice4(dk, b, h0 / chunk), sdv = slice4(dv, b, h0 / chunk),
+                       sdq = slice4(dq, b, h0);
+        const int64_t row = (b * H + h0) * M;
+        check(fa_bwd_dkdv_ds(type, &sq, &sk, &sv, &sg, f32(L) + row, f32(delta) + row, &sdk, &sdv, chunk,
+                             ds.mutable_data_ptr(), ds.numel(), 1, n, kn, M, N, D, c.causal, scale, p, c.seed,
+                             c.offset + (uint64_t)row * (uint64_t)N, stream), "fa_bwd_dkdv_ds");
+        check(fa_bwd_dq_from_ds(type, &sk, ds.const_data_ptr(), ds.numel(), &sdq, 1, n, kn, M, N, D, c.causal, scale,
+                                stream), "fa_bwd_dq_from_ds");
+      }
+  }
+  if (slices > Hk) {   // the kernel summed `chunk` heads of every group; add the chunks
+    dk = dk.view({B, Hk, slices / Hk, N, D}).sum(2);
+    dv = dv.view({B, Hk, slices / Hk, N, D}).sum(2);
+  }
+  return {dq, dk, dv};
+}
+
+template <class Call>
+struct Held : torch::CustomClassHolder {   // a call's parameters as one saved value of the autograd context
+  explicit Held(const Call& c) : call(c) {}
+  Call call;
+};
+template <class Call>
+void hold(AutogradContext* ctx, const Call& c) {
+  ctx->saved_data["call"] = c10::IValue::make_capsule(c10::make_intrusive<Held<Call>>(c));
+}
+template <class Call>
+const Call& held(AutogradContext* ctx) {
+  return static_cast<Held<Call>*>(ctx->saved_data["call"].toCapsule().get())->call;
+}
+
+struct FlashNode : torch::autograd::Function<FlashNode> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q0, const Tensor& k0, const Tensor& v0,
+                               const FlashCall& c, const FlashPlan& plan) {
+    const Tensor q = kernel_ready(q0), k = kernel_ready(k0), v = kernel_ready(v0);
+    variable_list out = flash_forward(q, k, v, c, plan);
+    ctx->save_for_backward({q, k, v, out[0], out[1]});
+    hold(ctx, c);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const FlashCall& c = held<FlashCall>(ctx);
+    const Tensor &q = saved[0], &k = saved[1];
+    const c10::DeviceGuard guard(q.device());
+    const int64_t limit = backward_settings(g_flash_settings, q.size(0), q.size(1), q.size(2), k.size(2), q.size(3), c.causal);
+    variable_list r = flash_backward(q, k, saved[2], saved[3], saved[4], grads[0], c, limit);
+    return {r[0], r[1], r[2], Tensor(), Tensor()};
+  }
+};
+
+bool needs_grad(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t->requires_grad()) return true;
+  return false;
+}
+
+PyObject* not_taken() { Py_RETURN_NOTIMPLEMENTED; }
+
+// flash(q, k, v, causal, sm_scale or None, dropout_p, return_log_normalizer, return_total_attention, return_seed_offset)
+PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 9, "flash: nine arguments");
+  if (!THPVariable_Check(a[0]) || !THPVariable_Check(a[1]) || !THPVariable_Check(a[2])) return not_taken();
+  const Tensor &q = THPVariable_Unpack(a[0]), &k = THPVariable_Unpack(a[1]), &v = THPVariable_Unpack(a[2]);
+  FlashCall c = {};
+  const int causal = PyObject_IsTrue(a[3]), want_lse = PyObject_IsTrue(a[6]), want_total = PyObject_IsTrue(a[7]),
+            want_seed = PyObject_IsTrue(a[8]);
+  if (causal < 0 || want_lse < 0 || want_total < 0 || want_seed < 0) throw python_error();
+  if (!is_operand(q, q) || !is_operand(k, q) || !is_operand(v, q) || !type_ok(q)) return not_taken();
+  const int64_t B = q.size(0), H = q.size(1), M = q.size(2), D = q.size(3), Hk = k.size(1), N = k.size(2);
+  if (!fits_int({B, H, M, N, Hk}) || k.size(0) != B || v.sizes() != k.sizes() || k.size(3) != D || H % Hk ||
+      !(D == 16 || D == 32 || D == 64 || D == 128))
+    return not_taken();
+  c.causal = causal;
+  c.want_total = want_total;
+  c.scale = a[4] == Py_None ? 1.0 / std::sqrt((double)D) : PyFloat_AsDouble(a[4]);
+  c.dropout_p = PyFloat_AsDouble(a[5]);
+  if (PyErr_Occurred()) { PyErr_Clear(); return not_taken(); }
+  if (!(c.dropout_p >= 0.0 && c.dropout_p < 1.0)) return not_taken();
+  const bool dropout = c.dropout_p > 0;
+
+  variable_list out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const c10::DeviceGuard guard(q.device());
+    FlashPlan plan;
+    // (a copy made for the kernels has unit-stride rows, so only a tensor used as it is can have distant rows)
+    const int64_t row_bytes = 2 * std::max(is_kernel_ready(k) ? k.stride(2) : D, is_kernel_ready(v) ? v.stride(2) : D);
+    const bool fine = plan_flash(plan, B, H, Hk, M, N, D, dropout, c.scale, row_bytes, fa_num_cus());
+    if (fine) {
+      if (dropout) {   // one Philox counter value per score element, from the device's default generator
+        at::Generator gen = at::globalContext().defaultGenerator(q.device());
+        std::lock_guard<std::mutex> lock(gen.mutex());
+        c.seed = gen.current_seed();
+        c.offset = gen.get_offset();
+        gen.set_offset(c.offset + (uint64_t)((B * H * M * N + 3) / 4 * 4));
+      }
+      if (needs_grad({&q, &k, &v})) out = FlashNode::apply(q, k, v, c, plan);
+      else out = flash_forward(kernel_ready(q), kernel_ready(k), kernel_ready(v), c, plan);
+    }
+  }
+  if (out.empty()) return not_taken();
+  if (!(want_lse || want_total || want_seed)) return THPVariable_Wrap(out[0]);
+  PyObject* r = PyTuple_New(5);
+  if (!r) throw python_error();
+  auto none = [] { Py_INCREF(Py_None); return Py_None; };
+  const bool seeded = dropout && want_seed;
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(out[0]));
+  PyTuple_SET_ITEM(r, 1, want_lse ? THPVariable_Wrap(out[1]) : none());
+  PyTuple_SET_ITEM(r, 2, want_total ? THPVariable_Wrap(out[2]) : none());
+  PyTuple_SET_ITEM(r, 3, seeded ? PyLong_FromLongLong((long long)c.seed) : none());
+  PyTuple_SET_ITEM(r, 4, seeded ? PyLong_FromLongLong((long long)c.offset) : none());
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// -------------------------------------------------------------------------------------- piecewise attention ----
+struct PiecewiseCall {
+  bool causal;
+  int w;
+  double scale;
+};
+
+struct PiecewiseNode : torch::autograd::Function<PiecewiseNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q1, const Tensor& k1, const Tensor& q2, const Tensor& k2,
+                        const Tensor& v, const PiecewiseCall& c) {
+    const Tensor ins[5] = {kernel_ready(q1), kernel_ready(k1), kernel_ready(q2), kernel_ready(k2), kernel_ready(v)};
+    Tensor L;
+    Tensor o = run(ins, c, L);
+    ctx->save_for_backward({ins[0], ins[1], ins[2], ins[3], ins[4], o, L});
+    hold(ctx, c);
+    return o;
+  }
+  static Tensor run(const Tensor* t, const PiecewiseCall& c, Tensor& L) {
+    const int B = (int)t[0].size(0), H = (int)t[0].size(1), M = (int)t[0].size(2), D = (int)t[0].size(3), N = (int)t[1].size(2);
+    Tensor o = empty_result(t[0]);
+    L = empty({B, H, M}, at::kFloat, t[0]);
+    const fa_view4 a = view4(t[0]), b = view4(t[1]), x = view4(t[2]), y = view4(t[3]), v = view4(t[4]), vo = view4(o);
+    check(pw_fwd(dtype_code(o), &a, &b, &x, &y, &v, &vo, f32(L), B, H, M, N, D, c.w, c.causal, (float)c.scale,
+                 stream_of(o)), "pw_fwd");
+    return o;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto t = ctx->get_saved_variables();
+    const PiecewiseCall& c = held<PiecewiseCall>(ctx);
+    const Tensor &q1 = t[0], &k1 = t[1], &q2 = t[2], &k2 = t[3], &v = t[4], &o = t[5], &L = t[6];
+    const int B = (int)q1.size(0), H = (int)q1.size(1), M = (int)q1.size(2), D = (int)q1.size(3), N = (int)k1.size(2);
+    const c10::DeviceGuard guard(q1.device());
+    const int64_t limit = backward_settings(g_piecewise_settings, B, H, M, N, D, c.causal);
+    const Tensor g = kernel_ready(grads[0]);
+    const int type = dtype_code(q1);
+    const float scale = (float)c.scale;
+    void* stream = stream_of(q1);
+    Tensor delta = empty(L.sizes(), at::kFloat, q1);
+    const fa_view4 vo = view4(o), vg = view4(g);
+    check(fa_bwd_delta(type, &vo, &vg, f32(delta), B, H, M, D, stream), "fa_bwd_delta");
+    Tensor dq1 = empty(q1.sizes(), q1.scalar_type(), q1), dq2 = empty(q2.sizes(), q1.scalar_type(), q1);
+    Tensor dk1 = empty(k1.sizes(), q1.scalar_type(), q1), dk2 = empty(k2.sizes(), q1.scalar_type(), q1);
+    Tensor dv = empty(v.sizes(), q1.scalar_type(), q1);
+    // dS handed from the dK/dV kernel to the dQ kernels, one chunk grid per regime, when it pays
+    int64_t heads = ds_heads_per_launch(B, H, 1, M, N, D, limit, 2);
+    Tensor ds;
+    int64_t nb = B, step = H;   // batch entries and heads per launch
+    if (heads >= (int64_t)B * H) ds = ds_workspace(q1, B, H, M, N, 2);
+    else if (heads > 0) ds = ds_workspace(q1, nb = 1, step = std::min<int64_t>(heads, H), M, N, 2);
+    if (!ds.defined()) { nb = B; step = H; }
+    for (int64_t b = 0; b < B; b += nb)
+      for (int64_t h0 = 0; h0 < H; h0 += step) {
+        const int n = (int)(std::min<int64_t>(H, h0 + step) - h0);
+        auto at_slice = [&](const Tensor& x) { return slice4(x, b, h0); };
+        const fa_view4 a = at_slice(q1), bk = at_slice(k1), x = at_slice(q2), y = at_slice(k2), vv = at_slice(v),
+                       gg = at_slice(g), a1 = at_slice(dq1), b1 = at_slice(dk1), a2 = at_slice(dq2), b2 = at_slice(dk2),
+                       v1 = at_slice(dv);
+        const float *l = f32(L) + (b * H + h0) * M, *d = f32(delta) + (b * H + h0) * M;
+        if (ds.defined()) {
+          check(pw_bwd_dkdv_ds(type, &a, &bk, &x, &y, &vv, &gg, l, d, &b1, &b2, &v1, ds.mutable_data_ptr(), ds.numel(),
+                               (int)nb, n, M, N, D, c.w, c.causal, scale, stream), "pw_bwd_dkdv_ds");
+          check(pw_bwd_dq_from_ds(type, &bk, &y, ds.const_data_ptr(), ds.numel(), &a1, &a2, (int)nb, n, M, N, D, c.w,
+                                  c.causal, scale, stream), "pw_bwd_dq_from_ds");
+        } else {
+          check(pw_bwd_dkdv(type, &a, &bk, &x, &y, &vv, &gg, l, d, &b1, &b2, &v1, (int)nb, n, M, N, D, c.w, c.causal,
+                            scale, stream), "pw_bwd_dkdv");
+          check(pw_bwd_dq(type, &a, &bk, &x, &y, &vv, &gg, l, d, &a1, &a2, (int)nb, n, M, N, D, c.w, c.causal, scale,
+                          stream), "pw_bwd_dq");
+        }
+      }
+    return {dq1, dk1, dq2, dk2, dv, Tensor()};
+  }
+};
+
+// piecewise(q1, k1, q2, k2, v, dist_threshold, causal, sm_scale or None)
+PyObject* piecewise(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 8, "piecewise: eight arguments");
+  for (int i = 0; i < 5; ++i)
+    if (!THPVariable_Check(a[i])) return not_taken();
+  const Tensor &q1 = THPVariable_Unpack(a[0]), &k1 = THPVariable_Unpack(a[1]), &q2 = THPVariable_Unpack(a[2]),
+               &k2 = THPVariable_Unpack(a[3]), &v = THPVariable_Unpack(a[4]);
+  for (const Tensor* t : {&q1, &k1, &q2, &k2, &v})
+    if (!is_operand(*t, q1)) return not_taken();
+  const int64_t D = q1.size(3);
+  if (!type_ok(q1) || !fits_int({q1.size(0), q1.size(1), q1.size(2), k1.size(2)}) || q2.sizes() != q1.sizes() ||
+      k2.sizes() != k1.sizes() || v.sizes() != k1.sizes() || k1.size(0) != q1.size(0) || k1.size(1) != q1.size(1) ||
+      k1.size(3) != D || !(D == 16 || D == 32 || D == 64 || D == 128))
+    return not_taken();
+  const int causal = PyObject_IsTrue(a[6]);
+  if (causal < 0) throw python_error();
+  if (!PyLong_Check(a[5])) return not_taken();
+  int overflow = 0;
+  const long long w = PyLong_AsLongLongAndOverflow(a[5], &overflow);
+  if (overflow || w < INT32_MIN || w > INT32_MAX) return not_taken();
+  PiecewiseCall c = {causal != 0, (int)w, a[7] == Py_None ? 1.0 / std::sqrt((double)D) : PyFloat_AsDouble(a[7])};
+  if (PyErr_Occurred()) { PyErr_Clear(); return not_taken(); }
+  Tensor o;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const c10::DeviceGuard guard(q1.device());
+    if (needs_grad({&q1, &k1, &q2, &k2, &v})) {
+      o = PiecewiseNode::apply(q1, k1, q2, k2, v, c);
+    } else {
+      const Tensor ins[5] = {kernel_ready(q1), kernel_ready(k1), kernel_ready(q2), kernel_ready(k2), kernel_ready(v)};
+      Tensor L;
+      o = PiecewiseNode::run(ins, c, L);
+    }
+  }
+  return THPVariable_Wrap(o);
+  END_HANDLE_TH_ERRORS
+}
+
+// ------------------------------------------------------------------------------------------ paged attention ----
+bool row_ready(const Tensor& t) {   // a (num_seqs, heads, D) tensor the kernels read or write as it is
+  return t.stride(2) == 1 && !((uintptr_t)t.const_data_ptr() & 15) && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0;
+}
+
+// paged(query, key_cache, value_cache, context_lens, block_tables, attn_scale, max_context_len), the launch chosen here
+PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 7, "paged: seven arguments");
+  for (int i = 0; i < 5; ++i)
+    if (!THPVariable_Check(a[i])) return not_taken();
+  const Tensor &q = THPVariable_Unpack(a[0]), &kc = THPVariable_Unpack(a[1]), &vc = THPVariable_Unpack(a[2]),
+               &lens = THPVariable_Unpack(a[3]), &bt = THPVariable_Unpack(a[4]);
+  if (!q.is_cuda() || q.dim() != 3 || q.layout() != at::kStrided || !is_operand(kc, kc) || !is_operand(vc, kc) ||
+      kc.device() != q.device() || kc.scalar_type() != q.scalar_type() || !type_ok(q))
+    return not_taken();
+  const int64_t seqs = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = kc.size(1), block = kc.size(2);
+  if (!fits_int({seqs, Hq, Hkv, block}) || kc.size(3) != D || vc.sizes() != kc.sizes() || vc.strides() != kc.strides() ||
+      kc.stride(3) != 1 || Hq % Hkv || !(D == 16 || D == 32 || D == 64 || D == 128 || D == 256 || D == 512) || !row_ready(q))
+    return not_taken();
+  if (lens.scalar_type() != at::kInt || lens.device() != q.device() || lens.dim() != 1 || lens.size(0) != seqs || !lens.is_contiguous() ||
+      bt.device() != q.device() || bt.dim() != 2 || bt.size(0) != seqs || bt.stride(1) != 1 ||
+      !(bt.scalar_type() == at::kInt || bt.scalar_type() == at::kLong))
+    return not_taken();
+  const double scale = PyFloat_AsDouble(a[5]);
+  const long long longest = PyLong_Check(a[6]) ? PyLong_AsLongLong(a[6]) : -1;
+  if (PyErr_Occurred()) { PyErr_Clear(); return not_taken(); }
+  if (longest < 0) return not_taken();
+  Tensor out;
+  {
+    pybind11::gil_scoped_release no_gil;
+    const c10::DeviceGuard guard(q.device());
+    out = q.is_contiguous() ? empty(q.sizes(), q.scalar_type(), q) : at::empty_like(q);   // the caller's layout, when the kernels can write it
+    if (!row_ready(out)) out = empty(q.sizes(), q.scalar_type(), q);
+    const int type = dtype_code(q), wgs = balanced_workgroups(seqs, Hkv, Hq / Hkv, D, longest, fa_num_cus());
+    void* stream = stream_of(q);
+    if (wgs > 0) {
+      const int bytes = paged_attn_balanced_workspace(wgs, (int)D);
+      Tensor ws = empty({bytes / 4}, at::kFloat, q);
+      check(paged_attn_balanced(type, out.mutable_data_ptr(), out.stride(0), out.stride(1), q.const_data_ptr(), q.stride(0), q.stride(1),
+                                kc.const_data_ptr(), vc.const_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2),
+                                (const int32_t*)lens.const_data_ptr(), bt.const_data_ptr(), bt.scalar_type() == at::kLong,
+                                bt.stride(0), (float)scale, (int)seqs, (int)Hq, (int)Hkv, (int)D, (int)block,
+                                ws.mutable_data_ptr(), (int64_t)bytes / 4 * 4, wgs, stream), "paged_attn_balanced");
+    } else {
+      check(paged_attn(type, out.mutable_data_ptr(), out.stride(0), out.stride(1), q.const_data_ptr(), q.stride(0), q.stride(1),
+                       kc.const_data_ptr(), vc.const_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2),
+                       (const int32_t*)lens.const_data_ptr(), bt.const_data_ptr(), bt.scalar_type() == at::kLong,
+                       bt.stride(0), (float)scale, (int)seqs, (int)Hq, (int)Hkv, (int)D, (int)block, 0, 1, nullptr,
+                       nullptr, nullptr, stream), "paged_attn");
+    }
+  }
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// ------------------------------------------------------------------------------------------------- module ----
+// decisions(B, H, Hk, M, N, D, num_cus, ds_limit_mib) -> every launch decision for that shape, for the test that
+// holds them against the Python functions
+PyObject* decisions(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
+  long long B, H, Hk, M, N, D, cus, limit;
+  if (!PyArg_ParseTuple(args, "LLLLLLLL", &B, &H, &Hk, &M, &N, &D, &cus, &limit)) return nullptr;
+  const int c = (int)cus, splits = num_splits_heuristic(B, H, M, N, c, 128), chosen = choose_num_splits(B, H, Hk, M, N, c);
+  return Py_BuildValue("{s:i,s:i,s:i,s:i,s:i,s:L,s:L,s:i}", "num_splits_heuristic", splits, "choose_num_splits", chosen,
+                       "split_size", split_size(N, chosen), "wide_key_splits", wide_key_splits(B, H, M, N, D, c),
+                       "dkdv_heads_per_slice", dkdv_heads_per_slice(B, H, (int)(H / Hk), N, c), "ds_heads_per_launch",
+                       (long long)ds_heads_per_launch(B, H, (int)(H / Hk), M, N, D, limit, 1), "ds_heads_per_launch_piecewise",
+                       (long long)ds_heads_per_launch(B, H, 1, M, N, D, limit, 2), "balanced_workgroups",
+                       balanced_workgroups(B, Hk, H / Hk, D, N, c));
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(abi.check, flash settings, piecewise settings)
+PyObject* bind(PyObject*, PyObject* args) {
+  if (!PyArg_ParseTuple(args, "OOO", &g_check, &g_flash_settings, &g_piecewise_settings)) return nullptr;
+  for (PyObject* o : {g_check, g_flash_settings, g_piecewise_settings}) Py_INCREF(o);   // for the life of the process
+  Py_RETURN_NONE;
+}
+
+PyMethodDef kMethods[] = {
+    {"flash", (PyCFunction)(void*)flash, METH_FASTCALL, nullptr},
+    {"piecewise", (PyCFunction)(void*)piecewise, METH_FASTCALL, nullptr},
+    {"paged", (PyCFunction)(void*)paged, METH_FASTCALL, nullptr},
+    {"decisions", decisions, METH_VARARGS, nullptr},
+    {"bind", bind, METH_VARARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }

@@ -10,7 +10,7 @@ import os
 
 import torch
 
-from . import _abi, _config, _lib
+from . import _abi, _config, _lib, split_kv, total
 from .split_kv import num_splits_heuristic, split_kv_forward, split_units, DECODE_MAX_ROWS
 from .total import _total_attention
 from .dropout import philox_cuda_seed_offset
@@ -76,6 +76,21 @@ def get_bwd_config(B, H, M, N, D, causal):
     """(BLOCK_M, BLOCK_N, num_stages, num_warps) of the dK/dV kernel: queries per pipeline step, keys
     per workgroup (``flash.py:493-519`` hook, called as in ``flash.py:185-186``; see ``BWD_TILES``)."""
     return (64, 128, 2, 4)
+
+
+_STOCK_HOOKS = (get_fwd_config, split_kv.get_fwd_config, total.get_fwd_config)
+
+
+def _hooks_replaced():
+    """Whether a caller has replaced a tile-config hook that a forward calls (the backward's own hook is called
+    when a backward runs, by ``backward_settings``)."""
+    return (get_fwd_config, split_kv.get_fwd_config, total.get_fwd_config) != _STOCK_HOOKS
+
+
+def backward_settings(B, H, M, N, D, causal):
+    """What a backward reads when it runs: calls the tile hook and returns the dS workspace limit in MiB."""
+    _config.resolve(get_bwd_config, BWD_TILES, "flash_attention backward", (B, H, M, N, D, causal))
+    return DS_WORKSPACE_LIMIT_MIB
 
 
 def _check_arguments(q, k, v, dropout_p):
@@ -194,7 +209,7 @@ class FlashAttention(torch.autograd.Function):
         lib = _lib.get()
         do = _abi.kernel_ready(do)
         with torch.cuda.device(q.device):
-            _config.resolve(get_bwd_config, BWD_TILES, "flash_attention backward", (B, H, M, N, D, causal))
+            backward_settings(B, H, M, N, D, causal)
             delta = torch.empty_like(L)
             _abi.fa_bwd_delta(lib, o, do, delta)
             # dK/dV come out summed over each kv head's group of query heads (flash.py:205-206,250-251
@@ -299,7 +314,15 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
     the device's default generator and returned when ``return_seed_offset`` is set); it cannot be
     combined with a shape that takes the split-KV path, as in the reference.  With an empty batch, query
     or key axis nothing is launched: out is zero, the log-normalizer -inf, the total attention zero.
+
+    For GPU tensors the call is made in native code (``csrc/host.cpp``), which makes the same decisions as
+    ``FlashAttention`` below; that class serves replaced tile hooks and raises for arguments in error.
     """
+    if q.is_cuda and not _hooks_replaced():
+        out = _lib.native().flash(q, k, v, causal, sm_scale, dropout_p, return_log_normalizer,
+                                  return_total_attention, return_seed_offset)
+        if out is not NotImplemented:
+            return out
     if q.numel() == 0 or k.shape[2] == 0:
         _check_arguments(q, k, v, dropout_p)
         B, H, M, _ = q.shape

@@ -50,6 +50,10 @@ def attention(query, key_cache, value_cache, context_lens, block_tables, attn_sc
     head_size) with identical strides; context_lens (num_seqs,) of any integer type; block_tables (num_seqs,
     max_blocks_per_seq) int32 or int64.  Returns out shaped like ``query``; a sequence of context length
     0 gets a zero row."""
+    if num_splits == 0 and query.is_cuda:   # native host path (``csrc/host.cpp``); what it does not take is served below
+        out = _lib.native().paged(query, key_cache, value_cache, context_lens, block_tables, attn_scale, max_context_len)
+        if out is not NotImplemented:
+            return out
     num_seqs, num_q_heads, head_size = query.shape
     num_kv_heads, block_size = key_cache.shape[1], key_cache.shape[2]
     assert key_cache.shape[3] == head_size and value_cache.shape == key_cache.shape

@@ -8,7 +8,7 @@ import math
 
 import torch
 
-from . import _abi, _config, _lib
+from . import _abi, _config, _lib, flash
 from .flash import NothingToAttend, _ds_workspace, ds_heads_per_launch
 
 __all__ = ["attention"]
@@ -27,6 +27,15 @@ def get_fwd_config(B, H, M, N, D, causal):
 def get_bwd_config(B, H, M, N, D, causal):
     """The same for the dK/dV kernel (``piecewise.py:98-99, 373-405``; ``BWD_TILES``)."""
     return (64, 128, 2, 4)
+
+
+_STOCK_FWD_HOOK = get_fwd_config
+
+
+def backward_settings(B, H, M, N, D, causal):
+    """What a backward reads when it runs: calls the tile hook and returns the dS workspace limit in MiB."""
+    _config.resolve(get_bwd_config, BWD_TILES, "piecewise_attention backward", (B, H, M, N, D, causal))
+    return flash.DS_WORKSPACE_LIMIT_MIB
 
 
 class PiecewiseAttention(torch.autograd.Function):
@@ -58,8 +67,7 @@ class PiecewiseAttention(torch.autograd.Function):
         lib = _lib.get()
         do = _abi.kernel_ready(do)
         with torch.cuda.device(q1.device):
-            _config.resolve(get_bwd_config, BWD_TILES, "piecewise_attention backward",
-                            (q1.shape[0], q1.shape[1], q1.shape[2], k1.shape[2], q1.shape[3], ctx.causal))
+            backward_settings(q1.shape[0], q1.shape[1], q1.shape[2], k1.shape[2], q1.shape[3], ctx.causal)
             delta = torch.empty_like(L)
             _abi.fa_bwd_delta(lib, o, do, delta)
             dk1 = torch.empty(k1.shape, dtype=k1.dtype, device=k1.device)
@@ -101,6 +109,10 @@ def attention(q1, k1, q2, k2, v, dist_threshold, causal=False, sm_scale=None):
     of query m and key n is ``q2[m].k2[n]`` when the signed distance ``m + seqlen_k - seqlen_q - n``
     is at least ``dist_threshold`` and ``q1[m].k1[n]`` otherwise.  Returns out (batch, heads,
     seqlen_q, headdim); zero when the batch, query or key axis is empty (nothing is launched)."""
+    if q1.is_cuda and get_fwd_config is _STOCK_FWD_HOOK:   # native host path, as in ``flash.attention``
+        out = _lib.native().piecewise(q1, k1, q2, k2, v, dist_threshold, causal, sm_scale)
+        if out is not NotImplemented:
+            return out
     if q1.numel() == 0 or k1.shape[2] == 0:
         assert q1.shape == q2.shape and k1.shape == k2.shape == v.shape and q1.shape[-1] == k1.shape[-1]
         return NothingToAttend.apply(q1, k1, q2, k2, v)
