@@ -39,6 +39,7 @@ struct DecCfg {
   static constexpr int NDB = D / 16;          // 16-wide slices of the output
   static constexpr int CPR = D / 8;           // 16-byte chunks per row
   static constexpr int CH = (TK * CPR + 63) / 64;  // chunks per lane per step
+  static constexpr int RPI = 64 / CPR;             // rows per load instruction
   static constexpr int NSETS = 1;   // register sets of loads in flight
   static constexpr int K_LD = DK + 8;
   static constexpr int V_LD = D + 32;  // 64 B of padding: the 4 rows of a transposing read fall in disjoint banks
@@ -63,13 +64,30 @@ struct DecodeOut {
   float row_sum[kPerThread];  // sum_j exp(scale * (s_j - row_max))
 };
 
-// Src must provide:
-//   struct Ids;                                             per-lane lookup state for one step
-//   void lookup(Ids&, int n0, int n_end, int lane) const;   start resolving the rows of the step at key n0
+// The thread index for addressing results: what is derived from it is formed behind the loop over the keys.  Derived
+// from the index itself it would be formed before the loop (in the balanced paged kernel, before the loop over pairs)
+// and, past the 256 registers, go to scratch memory and back.
+FA_DEVICE int thread_for_output() {
+  uint32_t t = (uint32_t)hw::thread_id();
+  hw::pin(t);
+  return (int)t;
+}
+
+// A load instruction of a step covers RPI consecutive keys (64 lanes of 16 bytes).  Src must provide:
+//   struct Ids;                                             lookup state for one step
+//   void lookup(Ids&, int n0, int n_last, int lane) const;  start resolving the rows of the step at key n0 (at most n_last)
 //   const T* k_row(const Ids&, int i, int n) const;         row pointer of key n (chunk slot i of the lane)
 //   const T* v_row(const Ids&, int i, int n) const;
+// and, with kUniform (the RPI keys of an instruction lie k_stride() bytes apart: every layout but unusual block sizes),
+//   void resolve(Ids&, int n0, int lane) const;             before the first base of a step whose TK keys all exist
+//   const T* k_base(const Ids&, int i, int n0) const;       row of the first key of instruction i of that step: one
+//   const T* v_base(const Ids&, int i, int n0) const;       address in scalar registers for all lanes
+// An address per lane and load costs 20 vector instructions and two registers each, 16 times per step; with a scalar
+// base and a constant lane offset a step's loads take two to four scalar instructions each.  The last step of a range
+// may be incomplete and takes the addresses per lane.
+// n_rows: the query rows of the workgroup that exist (the same in every lane); only those are merged and valid in out.
 template <class T, int D, class Src>
-FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane % 16, or nullptr */,
+FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane % 16, or nullptr */, int n_rows,
                             int n_begin, int n_end, int lane_limit /* keys n < lane_limit are visible */,
                             float c2, unsigned char* smem, DecodeOut<D>& out) {
   using C = DecCfg<T, D>;
@@ -108,8 +126,9 @@ FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane 
   for (int i = 0; i < C::NDB; ++i) oacc[i] = hw::f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int total_tiles = n_end > n_begin ? cdiv(n_end - n_begin, C::TK) : 0;
-  const int my_tiles = total_tiles > wave ? (total_tiles - wave + 3) / 4 : 0;
-  auto tile_start = [&](int j) { return n_begin + (wave + 4 * j) * C::TK; };
+  const int wave_s = hw::uniform(wave);   // the loop over the steps is a scalar one
+  const int my_tiles = total_tiles > wave_s ? (total_tiles - wave_s + 3) / 4 : 0;
+  auto tile_start = [&](int j) { return n_begin + (wave_s + 4 * j) * C::TK; };
 
   u32x4 kst0[C::CH], vst0[C::CH];
   u32x4 kst1[C::NSETS == 2 ? C::CH : 1], vst1[C::NSETS == 2 ? C::CH : 1];
@@ -123,6 +142,19 @@ FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane 
   // positions (flash.py:448-461, split_kv.py:137), so a non-finite value there gives NaN in both.
   static_assert(C::TK * C::CPR == 64 * C::CH, "a step is a whole number of 64-lane load instructions");
   auto fetch = [&](int n0, u32x4* kst, u32x4* vst) {
+    if constexpr (Src::kUniform) {
+      if (n0 + C::TK <= n_end) {
+        const uint32_t row = (uint32_t)(lane / C::CPR), col = (uint32_t)(lane % C::CPR) * 16u;
+        const uint32_t k_off = row * src.k_stride() + col, v_off = row * src.v_stride() + col;
+        src.resolve(ids, n0, lane);
+#pragma unroll
+        for (int i = 0; i < C::CH; ++i) {
+          kst[i] = *(const u32x4*)((const char*)src.k_base(ids, i, n0) + k_off);
+          vst[i] = *(const u32x4*)((const char*)src.v_base(ids, i, n0) + v_off);
+        }
+        return;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < C::CH; ++i) {
       const int c = lane + 64 * i;
@@ -144,14 +176,14 @@ FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane 
 
   // loads of the first NSETS steps, and the block-table rows of the step after them
   if (my_tiles > 0) {
-    src.lookup(ids, tile_start(0), n_end, lane);
+    src.lookup(ids, tile_start(0), n_end - 1, lane);
     fetch(tile_start(0), kst0, vst0);
   }
   if (C::NSETS == 2 && my_tiles > 1) {
-    src.lookup(ids, tile_start(1), n_end, lane);
+    src.lookup(ids, tile_start(1), n_end - 1, lane);
     fetch(tile_start(1), kst1, vst1);
   }
-  if (my_tiles > C::NSETS) src.lookup(ids, tile_start(C::NSETS), n_end, lane);
+  if (my_tiles > C::NSETS) src.lookup(ids, tile_start(C::NSETS), n_end - 1, lane);
 
   auto step = [&](int j, u32x4* kst, u32x4* vst) {
     const int n0 = tile_start(j);
@@ -159,7 +191,7 @@ FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane 
     commit(kst, vst);
     if (j + C::NSETS < my_tiles) {
       fetch(tile_start(j + C::NSETS), kst, vst);
-      if (j + C::NSETS + 1 < my_tiles) src.lookup(ids, tile_start(j + C::NSETS + 1), n_end, lane);
+      if (j + C::NSETS + 1 < my_tiles) src.lookup(ids, tile_start(j + C::NSETS + 1), n_end - 1, lane);
     }
     hw::wave_sync();
 
@@ -256,7 +288,7 @@ FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane 
   hw::block_sync();  // every wavefront is done with its staging patch
   float* area = (float*)smem;
   constexpr int RS = D + 2;
-  {
+  if (li < n_rows) {
     float* mine = area + (wave * C::ROWS + li) * RS;
 #pragma unroll
     for (int db = 0; db < C::NDB; ++db)
@@ -265,24 +297,27 @@ FA_DEVICE void decode_block(const Src& src, const T* q_row /* query row of lane 
     if (g == 0) { mine[D] = m_i; mine[D + 1] = l_i; }
   }
   hw::block_sync();
+  const int out_tid = thread_for_output();
 #pragma unroll
   for (int e = 0; e < DecodeOut<D>::kPerThread; ++e) {
-    const int idx = tid + e * kThreads;
-    const int row = (idx / D) % C::ROWS, d = idx % D;  // idx >= 16 * D occurs only when 16 * D < 256; callers skip it
-    float mw[4], mm = neg_inf();
+    if (e * kThreads / D < n_rows) {   // uniform: a GQA group of 4 reads a quarter of the area
+      const int idx = out_tid + e * kThreads;
+      const int row = (idx / D) % C::ROWS, d = idx % D;  // idx >= 16 * D occurs only when 16 * D < 256; callers skip it
+      float mw[4], mm = neg_inf();
 #pragma unroll
-    for (int w = 0; w < 4; ++w) { mw[w] = area[(w * C::ROWS + row) * RS + D]; mm = fmaxf(mm, mw[w]); }
-    const float m_use = (mm == neg_inf()) ? 0.f : mm;
-    float acc = 0.f, sum = 0.f;
+      for (int w = 0; w < 4; ++w) { mw[w] = area[(w * C::ROWS + row) * RS + D]; mm = fmaxf(mm, mw[w]); }
+      const float m_use = (mm == neg_inf()) ? 0.f : mm;
+      float acc = 0.f, sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float f = hw::exp2_fast((mw[w] - m_use) * c2);  // -inf -> 0
-      acc += f * area[(w * C::ROWS + row) * RS + d];
-      sum += f * area[(w * C::ROWS + row) * RS + D + 1];
+      for (int w = 0; w < 4; ++w) {
+        const float f = hw::exp2_fast((mw[w] - m_use) * c2);  // -inf -> 0
+        acc += f * area[(w * C::ROWS + row) * RS + d];
+        sum += f * area[(w * C::ROWS + row) * RS + D + 1];
+      }
+      out.o[e] = acc;
+      out.row_max[e] = mm;
+      out.row_sum[e] = sum;
     }
-    out.o[e] = acc;
-    out.row_max[e] = mm;
-    out.row_sum[e] = sum;
   }
 }
 

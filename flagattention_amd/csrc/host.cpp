@@ -80,8 +80,9 @@ int num_splits_heuristic(int64_t B, int64_t H, int64_t M, int64_t N, int cus, in
 // split_kv.choose_num_splits
 int choose_num_splits(int64_t B, int64_t H, int64_t Hk, int64_t M, int64_t N, int cus) {
   const int64_t base = B * Hk * cdiv(H / Hk * M, 16), units = cdiv(N, kSplitBlockN);
-  const int64_t want = cdiv(2 * (int64_t)cus, base), cap = std::max<int64_t>(1, N / 512);
-  int64_t splits = std::min(std::max<int64_t>(1, std::min<int64_t>({want, cap, 128})), units);
+  int64_t splits = std::min(cdiv(2 * (int64_t)cus, base), std::max<int64_t>(1, N / 512));
+  if (N >= 1024) splits = std::max(splits, std::min(cdiv(cus, base), N / 128));
+  splits = std::min<int64_t>({splits, 128, units});
   while (splits > 1 && cdiv(units, splits) * (splits - 1) >= units) --splits;
   return (int)splits;
 }

@@ -129,6 +129,21 @@ FA_DEVICE uint64_t ballot(bool pred) { return __builtin_amdgcn_ballot_w64(pred);
 // Value held by lane l - delta (lanes below delta keep their own), and by a given lane.
 FA_DEVICE int shfl_up(int x, int delta) { return __shfl_up(x, delta, 64); }
 FA_DEVICE int lane_value(int x, int lane) { return __shfl(x, lane, 64); }
+// Inclusive prefix sum over the 64 lanes: data-parallel-primitive adds inside the rows of 16 lanes, then each row's
+// total into the rows behind it -- six vector instructions, where exchanges through LDS cost a latency each.
+FA_DEVICE int wave_prefix_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 (nothing shifts in: + 0)
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return x;
+}
+// Value of lane 63, as a scalar.
+FA_DEVICE int last_lane(int x) { return __builtin_amdgcn_readlane(x, 63); }
+// Value of a lane whose index is the same in every lane, as a scalar.
+FA_DEVICE int read_lane(int x, int lane) { return __builtin_amdgcn_readlane(x, lane); }
 
 // Value held by lane (l ^ 32).
 FA_DEVICE float xor32(float x) { return __shfl_xor(x, 32, 64); }

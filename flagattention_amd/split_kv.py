@@ -74,16 +74,19 @@ def choose_num_splits(B, H, Hk, M, N, num_cus, reference_splits):
     ``B * Hk * ceil(G * M / 16)`` workgroups per split -- fewer than the per-query-head grid the
     reference's rule assumes.  Splits are added until the launch has about two workgroups per
     compute unit -- one resident wave, which measures 2-15 % faster than two shorter waves -- as long
-    as every piece keeps at least 512 keys (four 32-key steps per wavefront).
+    as every piece keeps at least 512 keys (four 32-key steps per wavefront).  From 1024 keys on, until
+    it has one workgroup per compute unit, a piece may be as short as 128 keys, one step per wavefront
+    (1024 keys, 8 workgroups per split: split and merge 10.8 us in two pieces, 7.3 in eight; a launch
+    that small is a chain of latencies, and every further step adds 1 us to it).
     ``reference_splits`` (the count the reference's rule gives) is not used beyond having selected the
     split path.  The result of the operator does not depend on the count."""
     group = H // Hk
     base = B * Hk * -(-(group * M) // 16)
     n_units = -(-N // SPLIT_BLOCK_N)
-    want = -(-2 * num_cus // base)
-    cap = max(1, N // 512)
-    splits = max(1, min(want, cap, 128))
-    splits = min(splits, n_units)
+    splits = min(-(-2 * num_cus // base), max(1, N // 512))
+    if N >= 1024:
+        splits = max(splits, min(-(-num_cus // base), N // 128))
+    splits = min(splits, 128, n_units)
     # drop counts that would leave the last piece empty
     while splits > 1 and (-(-n_units // splits)) * (splits - 1) >= n_units:
         splits -= 1

@@ -326,6 +326,13 @@ inline int shfl_up(int x, int delta) {
   }
   return result;
 }
+inline int wave_prefix_sum(int x) {
+  for (int d = 1; d < 64; d <<= 1) {
+    const int t = shfl_up(x, d);
+    if ((hwsim::cur & 63) >= d) x += t;
+  }
+  return x;
+}
 inline int lane_value(int x, int lane) {
   int result = x;
   const int me = hwsim::cur & 63;
@@ -335,6 +342,10 @@ inline int lane_value(int x, int lane) {
   }
   return result;
 }
+inline int read_lane(int x, int lane) {   // in halves: lane_value() passes through a float
+  return (int)((uint32_t)lane_value((int)((uint32_t)x >> 16), lane) << 16 | (uint32_t)lane_value(x & 0xffff, lane));
+}
+inline int last_lane(int x) { return lane_value(x, 63); }
 inline uint64_t ballot(bool pred) {
   uint64_t mask = 0;
   const int me = hwsim::cur & 63;
