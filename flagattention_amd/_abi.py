@@ -88,6 +88,33 @@ def fa_fwd(lib, q, k, v, o, lse, causal, sm_scale, dropout=NO_DROPOUT, block_m=0
                      _u64(dropout[2]), int(block_m), stream_of(q)), "fa_fwd")
 
 
+def fa_fwd_keep(lib, q, k, v, o, lse, keep, causal, sm_scale, dropout):
+    """Forward with dropout that leaves its mask in ``keep`` (int32, B * H * fa_dropout_keep_words(M, N))."""
+    B, H, M, D = q.shape
+    Hk, N = k.shape[1], k.shape[2]
+    assert keep.numel() >= B * H * lib.fa_dropout_keep_words(M, N)
+    check(lib.fa_fwd_keep(dtype_code(q), view4(q), view4(k), view4(v), view4(o), ptr(lse), ptr(keep), B, H, Hk, M, N, D,
+                          int(causal), float(sm_scale), float(dropout[0]), _u64(dropout[1]), _u64(dropout[2]),
+                          stream_of(q)), "fa_fwd_keep")
+
+
+def fa_bwd_dkdv_keep(lib, q, k, v, do, lse, delta, dk, dv, ds, keep, causal, sm_scale, dropout_p):
+    B, H, M, D = q.shape
+    Hk, N = k.shape[1], k.shape[2]
+    check(lib.fa_bwd_dkdv_keep(dtype_code(q), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta), view4(dk),
+                               view4(dv), ptr(ds), 0 if ds is None else ds.numel() * ds.element_size(), ptr(keep),
+                               B, H, Hk, M, N, D, int(causal), float(sm_scale), float(dropout_p), stream_of(q)),
+          "fa_bwd_dkdv_keep")
+
+
+def fa_bwd_dq_keep(lib, q, k, v, do, lse, delta, dq, keep, causal, sm_scale, dropout_p):
+    B, H, M, D = q.shape
+    Hk, N = k.shape[1], k.shape[2]
+    check(lib.fa_bwd_dq_keep(dtype_code(q), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta), view4(dq),
+                             ptr(keep), B, H, Hk, M, N, D, int(causal), float(sm_scale), float(dropout_p),
+                             stream_of(q)), "fa_bwd_dq_keep")
+
+
 def pw_fwd(lib, q1, k1, q2, k2, v, o, lse, w, causal, sm_scale):
     B, H, M, D = q1.shape
     N = k1.shape[2]

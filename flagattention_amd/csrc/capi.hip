@@ -71,6 +71,32 @@ int fa_fwd(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, c
   return fa::run_fwd(p, false, (hipStream_t)stream);
 }
 
+int fa_dropout_keep_words(int M, int N) {
+  if (M <= 0 || N <= 0) return FA_ERR_BAD_ARGUMENT;
+  const int64_t words = fa::dropout_keep_words(M, N);
+  return words > 0x7fffffff ? FA_ERR_UNSUPPORTED : (int)words;
+}
+
+static bool keep_ok(const uint32_t* keep, float dropout_p) {
+  return keep && !(((uintptr_t)keep) & 3) && dropout_p > 0.f && dropout_p < 1.f;
+}
+
+int fa_fwd_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* o, float* lse,
+                uint32_t* keep, int B, int H, int Hk, int M, int N, int D, int causal, float sm_scale, float dropout_p,
+                uint64_t seed, uint64_t offset, void* stream) {
+  if (!view_ok(q) || !view_ok(k) || !view_ok(v) || !view_ok(o) || !lse || !keep_ok(keep, dropout_p)) return FA_ERR_BAD_ARGUMENT;
+  if (!head_dim_ok(D)) return FA_ERR_UNSUPPORTED;
+  if (Hk <= 0 || H % Hk) return FA_ERR_BAD_ARGUMENT;
+  fa::FwdParams p = {};
+  p.q = to_view(q); p.k = to_view(k); p.v = to_view(v); p.o = to_view(o);
+  p.lse = lse; p.keep = keep;
+  p.B = B; p.H = H; p.M = M; p.N = N; p.D = D;
+  p.group = H / Hk;
+  p.causal = causal; p.sm_scale = sm_scale; p.dtype = dtype;
+  p.dropout_p = dropout_p; p.seed = seed; p.offset = offset;
+  return fa::run_fwd(p, false, (hipStream_t)stream);
+}
+
 int pw_fwd(int dtype, const fa_view4* q1, const fa_view4* k1, const fa_view4* q2, const fa_view4* k2,
            const fa_view4* v, const fa_view4* o, float* lse, int B, int H, int M, int N, int D,
            int dist_threshold, int causal, float sm_scale, void* stream) {
@@ -135,6 +161,33 @@ int fa_bwd_dq(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v
   if (!view_ok(dq)) return FA_ERR_BAD_ARGUMENT;
   p.dq = to_view(dq);
   p.dropout_p = dropout_p; p.seed = seed; p.offset = offset;
+  return fa::run_bwd_dq(p, false, (hipStream_t)stream);
+}
+
+int fa_bwd_dkdv_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* dout,
+                     const float* lse, const float* delta, const fa_view4* dk, const fa_view4* dv, void* ds_workspace,
+                     int64_t ds_workspace_bytes, const uint32_t* keep, int B, int H, int Hk, int M, int N, int D,
+                     int causal, float sm_scale, float dropout_p, void* stream) {
+  fa::BwdParams p = {};
+  int rc = fill_bwd(p, dtype, q, k, v, dout, lse, delta, B, H, Hk, M, N, D, causal, sm_scale);
+  if (rc) return rc;
+  if (!view_ok(dk) || !view_ok(dv) || !keep_ok(keep, dropout_p)) return FA_ERR_BAD_ARGUMENT;
+  if (ds_workspace && ((((uintptr_t)ds_workspace) & 15) || ds_workspace_bytes < fa::bwd_ds_workspace_bytes(B, H, M, N)))
+    return FA_ERR_BAD_ARGUMENT;
+  p.dk = to_view(dk); p.dv = to_view(dv);
+  p.chunk = 1; p.dropout_p = dropout_p; p.keep = keep; p.ds = ds_workspace;
+  return ds_workspace ? fa::run_bwd_dkdv_ds(p, false, (hipStream_t)stream) : fa::run_bwd_dkdv(p, false, (hipStream_t)stream);
+}
+
+int fa_bwd_dq_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* dout,
+                   const float* lse, const float* delta, const fa_view4* dq, const uint32_t* keep, int B, int H, int Hk,
+                   int M, int N, int D, int causal, float sm_scale, float dropout_p, void* stream) {
+  fa::BwdParams p = {};
+  int rc = fill_bwd(p, dtype, q, k, v, dout, lse, delta, B, H, Hk, M, N, D, causal, sm_scale);
+  if (rc) return rc;
+  if (!view_ok(dq) || !keep_ok(keep, dropout_p)) return FA_ERR_BAD_ARGUMENT;
+  p.dq = to_view(dq);
+  p.dropout_p = dropout_p; p.keep = keep;
   return fa::run_bwd_dq(p, false, (hipStream_t)stream);
 }
 

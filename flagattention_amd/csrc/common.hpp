@@ -171,27 +171,84 @@ FA_DEVICE typename hw::Elem<T>::v8 pack_half_block(const f32x16& s, int c) {
 // c = offset + ((b * H + h) * M + m) * N + n, key (lo(seed), hi(seed)), 6 rounds, first output word;
 // the word, read as int32 with negative values folded by -x - 1, times 4.6566127342e-10 is the
 // uniform number, and the probability is kept when it exceeds dropout_p.
-FA_DEVICE uint32_t philox6_first_word(uint32_t c0, uint32_t c1, uint32_t k0, uint32_t k1) {
-  uint32_t c2 = 0u, c3 = 0u;
+//
+// What the kernels draw with: of the four words and six rounds only what reaches the first word is formed, three-way
+// exclusive ors are one instruction, and the comparison is made on the integer (dropout_threshold below).  1.06e12 ->
+// 1.66e12 elements/s, 95 clocks per 64 elements, which is still two to three times what the rest of the attention
+// kernels does for them -- hence the mask goes from the forward to the backward as bits (KeepMask).
+constexpr uint32_t kPhiloxM0 = 0xD2511F53u, kPhiloxM1 = 0xCD9E8D57u, kPhiloxW0 = 0x9E3779B9u, kPhiloxW1 = 0xBB67AE85u;
+
+// The part of round 1 that depends on the counter's upper word alone.
+struct PhiloxUpper { uint32_t x2, x3; };
+FA_DEVICE PhiloxUpper philox_upper(uint32_t hi, uint32_t k0, uint32_t k1) {
+  const uint64_t p = (uint64_t)kPhiloxM0 * (hi ^ k0);
+  return PhiloxUpper{(uint32_t)(p >> 32) ^ (k1 + kPhiloxW1), (uint32_t)p};
+}
+FA_DEVICE uint32_t philox6_first_word(uint32_t lo, PhiloxUpper up, uint32_t k0, uint32_t k1) {
+  const uint64_t a0 = (uint64_t)kPhiloxM0 * lo;                               // round 0: words 2 and 3 are zero
+  const uint64_t b1 = (uint64_t)kPhiloxM1 * ((uint32_t)(a0 >> 32) ^ k1);      // round 1
+  uint32_t c0 = (uint32_t)(b1 >> 32) ^ (k0 + kPhiloxW0), c1 = (uint32_t)b1;
+  uint32_t c2 = up.x2 ^ (uint32_t)a0, c3 = up.x3;
 #pragma unroll
-  for (int round = 0; round < 6; ++round) {
-    const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0, n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+  for (int round = 2; round < 5; ++round) {
+    const uint64_t p0 = (uint64_t)kPhiloxM0 * c0, p1 = (uint64_t)kPhiloxM1 * c2;
+    c0 = hw::xor3((uint32_t)(p1 >> 32), c1, k0 + (uint32_t)round * kPhiloxW0);
+    c2 = hw::xor3((uint32_t)(p0 >> 32), c3, k1 + (uint32_t)round * kPhiloxW1);
     c1 = (uint32_t)p1;
     c3 = (uint32_t)p0;
-    c0 = n0;
-    c2 = n2;
-    k0 += 0x9E3779B9u;
-    k1 += 0xBB67AE85u;
   }
-  return c0;
+  return hw::xor3((uint32_t)(((uint64_t)kPhiloxM1 * c2) >> 32), c1, k0 + 5u * kPhiloxW0);
 }
-FA_DEVICE bool dropout_keeps(uint64_t counter, uint64_t seed, float dropout_p) {
-  const uint32_t x = philox6_first_word((uint32_t)counter, (uint32_t)(counter >> 32), (uint32_t)seed,
-                                        (uint32_t)(seed >> 32));
-  int32_t v = (int32_t)x;
-  v = v < 0 ? ~v : v;  // -v - 1
-  return (float)v * 4.6566127342e-10f > dropout_p;
+// The word x is kept when v = (x as int32, negative folded by -x - 1), times 4.6566127342e-10 in fp32, exceeds
+// dropout_p.  v -> (float)v * c is monotonic, so there is a smallest kept v, `threshold`; and the dropped words are
+// those of [-threshold, threshold), i.e. x + threshold < 2 threshold without sign.
+inline uint32_t dropout_threshold(float dropout_p) {
+  uint32_t lo = 0, hi = 0x7fffffffu;   // (float)hi * c > dropout_p for every dropout_p < 1 that fp32 tells from 1
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo) / 2;
+    const float u = (float)(int32_t)mid * 4.6566127342e-10f;
+    if (u > dropout_p) hi = mid;
+    else lo = mid + 1;
+  }
+  return lo;
+}
+FA_DEVICE bool dropout_keeps(uint64_t counter, uint64_t seed, uint32_t threshold) {
+  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+  return philox6_first_word((uint32_t)counter, philox_upper((uint32_t)(counter >> 32), k0, k1), k0, k1) + threshold >= 2u * threshold;
+}
+// Bits r = 0..15: whether the element at counter + block_row(r, 0) is kept (16 elements of a result block whose rows
+// run along the counter).
+FA_DEVICE uint32_t dropout_draw16(uint64_t counter, uint64_t seed, uint32_t threshold) {
+  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32), lo = (uint32_t)counter, hi = (uint32_t)(counter >> 32);
+  uint32_t bits = 0u;
+  if (hw::wave_any(lo > 0xffffffffu - 27u)) {   // the counter's upper word changes inside the block
+    hw::keep_branch();
+#pragma unroll 1
+    for (int r = 15; r >= 0; --r)
+      bits = 2u * bits + (dropout_keeps(counter + (uint64_t)(8 * (r >> 2) + (r & 3)), seed, threshold) ? 1u : 0u);
+    return bits;
+  }
+  const PhiloxUpper up = philox_upper(hi, k0, k1);
+#pragma unroll
+  for (int r = 15; r >= 0; --r)
+    hw::append_at_least(bits, philox6_first_word(lo + (uint32_t)(8 * (r >> 2) + (r & 3)), up, k0, k1) + threshold, 2u * threshold);
+  return bits;
+}
+
+// The mask of a forward as the backward reads it: one 32-bit word per query row and block of 32 keys (bit = key inside
+// the block), words of one key block contiguous along the rows.  Blocks that no row of a 32-row block sees under the
+// causal mask are neither written nor read.
+struct KeepMask {
+  int64_t rows, blocks;   // words per key block, key blocks per (batch, head)
+  FA_DEVICE KeepMask(int M, int N) : rows(32 * (int64_t)cdiv(M, 32)), blocks(2 * (int64_t)cdiv(N, 64)) {}
+  FA_DEVICE int64_t head(int64_t bh) const { return bh * blocks * rows; }
+  FA_DEVICE int64_t block(int kb) const { return (int64_t)(kb < blocks ? kb : blocks - 1) * rows; }
+};
+// The 16 bits a lane holds (keys block_row(r, half) of a block) in their places in the word.
+FA_DEVICE uint32_t keep_spread(uint32_t bits16, int half) {
+  uint32_t x = (bits16 | (bits16 << 8)) & 0x00ff00ffu;
+  x = (x | (x << 4)) & 0x0f0f0f0fu;
+  return x << (4 * half);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -67,7 +67,7 @@ int run_bwd_delta(const BwdParams& p, hipStream_t stream) {
 }
 
 // ------------------------------------------------------------------------------- dK and dV ----
-template <class T, int D, bool PW>
+template <class T, int D, bool PW, int DROP = 0>
 struct KvCfg {
   static constexpr int BN = 128;  // keys per workgroup (32 per wavefront)
   static constexpr int BM = 64;   // queries per pipeline step
@@ -77,10 +77,13 @@ struct KvCfg {
   static constexpr int TILE = BM * LD;
   // register budget the compiler may use: 256 registers (two wavefronts per SIMD) at the small head sizes; at 64
   // and 128 the slot-structured body gets all 512 (at 64 it needs 229, so two workgroups still share a CU)
-  static constexpr int WAVES_PER_SIMD = D < 64 ? 2 : 1;
+  // (with dropout the body is the phase-by-phase one, which leaves room for two again where the mask is not drawn)
+  static constexpr int WAVES_PER_SIMD = DROP == 1 ? 1 : (D < 64 || (D == 64 && DROP)) ? 2 : 1;
   // one wavefront per SIMD: overlap of matrix and element-wise work has to come from the instruction order
-  static constexpr bool SLOTTED = WAVES_PER_SIMD == 1 && BM == 64 && (D == 128 || D == 64);
-  static constexpr size_t STAGE_BYTES = 2 * TILE * sizeof(T) + 2 * BM * sizeof(float);  // Q, dO, L, delta
+  static constexpr bool SLOTTED = !DROP && WAVES_PER_SIMD == 1 && BM == 64 && (D == 128 || D == 64);
+  static constexpr size_t STATS = 2 * TILE * sizeof(T);   // byte offset of L and delta behind the Q and dO tiles
+  static constexpr size_t KEEP = STATS + 2 * BM * sizeof(float);   // and of the mask words of a dropout kernel
+  static constexpr size_t STAGE_BYTES = KEEP + (DROP == 2 ? kThreads * sizeof(uint32_t) : 0);
   // the slot-structured body writes the next tile into LDS and passes the barrier before its last
   // matrix instructions, which still read the current tile: three stages
   static constexpr int STAGES = SLOTTED ? 3 : 2;
@@ -98,15 +101,17 @@ struct KvCfg {
 // Chunks are indexed (batch * H + head, key block, query block); both counts padded to 4.
 //
 // DROP: dropout as in the reference (flash.py:697-721): dV takes the masked P and is scaled by
-// 1 / (1 - dropout_p); dP is masked and scaled likewise; dS = P (dP - delta) with the unmasked P.
+// 1 / (1 - dropout_p); dP is masked and scaled likewise; dS = P (dP - delta) with the unmasked P.  1: the mask is drawn
+// again; 2: it is read as the forward left it (p.keep; B=4 H=16 T=1024 D=64 causal: 84 -> 42 us), every wavefront's
+// 64 words of a tile by way of LDS.
 //
 // GROUPED: the workgroup walks more than one query head (see below); a separate instantiation,
 // because the extra loop level costs the single-head kernel 10 % through register allocation alone.
-template <class T, int D, bool PW, bool DS = false, bool DROP = false, bool GROUPED = false>
-FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PER_SIMD)) fa_bwd_dkdv_kernel(BwdParams p) {
+template <class T, int D, bool PW, bool DS = false, int DROP = 0, bool GROUPED = false>
+FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (KvCfg<T, D, PW, DROP>::WAVES_PER_SIMD)) fa_bwd_dkdv_kernel(BwdParams p) {
   static_assert(!(GROUPED && (PW || DROP)), "grouped accumulation is built for plain attention without dropout");
   static_assert(!(PW && DROP), "piecewise attention has no dropout");
-  using C = KvCfg<T, D, PW>;
+  using C = KvCfg<T, D, PW, DROP>;
   using V8 = typename hw::Elem<T>::v8;
   FA_LDS_DECL(smem);
 
@@ -167,16 +172,21 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PE
   gr.init(tid, p.dout.st);
   float l_reg = 0.f, d_reg = 0.f;
   int l_row = 0;
+  // DROP == 2: thread t carries the word of query t % 64 of the tile for key block t / 64 of the workgroup
+  const KeepMask keep_at(M, N);
+  const uint32_t* keep_src = nullptr;
+  uint32_t keep_reg = 0u;
   // In the instantiation with the slot-structured body, LDS holds -L / sm_scale and -delta per row:
   // the score and dP accumulators start from them, so that P = exp2(c2 (q.k - L / sm_scale)) and
   // dS = P (dO.v - delta) take one multiplication each in the slots.
-  constexpr bool FOLDED = C::SLOTTED && !DROP;
+  constexpr bool FOLDED = C::SLOTTED;
   const float inv_scale = 1.f / p.sm_scale;
   auto fetch_stats = [&](int m0) {
     l_row = m0 + (tid & (C::BM - 1));
     const int mc = imin(l_row, M - 1);
     l_reg = lse[mc];
     d_reg = dlt[mc];
+    if (DROP == 2) keep_reg = keep_src[mc];
   };
   auto fetch = [&](int m0) {
     const int rows = M - m0;
@@ -191,7 +201,8 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PE
     T* s = (T*)base;
     qr.template commit<C::LD>(s);
     gr.template commit<C::LD>(s + C::TILE);
-    float* f = (float*)(base + 2 * C::TILE * sizeof(T));
+    float* f = (float*)(base + C::STATS);
+    if (DROP == 2) ((uint32_t*)(base + C::KEEP))[tid] = keep_reg;
     // rows past M get L = +inf, hence P = 0
     if (tid < C::BM) {
       if constexpr (FOLDED) {  // what the accumulators of q.k and dO.v start from
@@ -248,7 +259,8 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PE
     ds_regime_stride = (int64_t)p.B * p.H * nkb * nqb * 1024;
     ds_row = ds_near;
   }
-  if (DROP) drop_col = p.offset + ((uint64_t)batch * p.H + head) * M * (uint64_t)N + (uint64_t)(my_n < N ? my_n : 0);
+  if (DROP == 2) keep_src = p.keep + keep_at.head((int64_t)batch * p.H + head) + keep_at.block(n0 / 32 + tid / C::BM);
+  if (DROP == 1) drop_col = p.offset + ((uint64_t)batch * p.H + head) * M * (uint64_t)N + (uint64_t)(my_n < N ? my_n : 0);
 #pragma unroll
   for (int ph = 0; ph < (PW ? 2 : 1); ++ph) {
     far_phase = PW && ph == 1;
@@ -613,6 +625,20 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PE
           drow[g] = *(const hw::f32x4*)(sDl + sb * 32 + 8 * g + 4 * hh);
         }
         f32x16 pr, ds;
+        u32x4 keep_words[4];
+        uint32_t drawn = 0u;
+        if (DROP == 2) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) keep_words[g] = *(const u32x4*)(base + C::KEEP + 4 * (wave * C::BM + sb * 32 + 8 * g + 4 * hh));
+        } else if (DROP) {
+#pragma unroll
+          for (int r = 15; r >= 0; --r)
+            drawn = 2u * drawn + (dropout_keeps(drop_col + (uint64_t)(mr0 + block_row(r, hh)) * N, p.seed, p.threshold) ? 1u : 0u);
+        }
+        // x if the element (query of register r, this lane's key) survived the dropout, else 0
+        auto survivor = [&](int r, float x) {
+          return DROP == 2 ? hw::keep_if_bit(x, keep_words[r >> 2][r & 3], l32) : hw::keep_if_bit(x, drawn, r);
+        };
         if (need_mask) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
@@ -624,9 +650,8 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PE
             pv = keep ? pv : 0.f;
             float pd = pv, dpv = dp[r];
             if (DROP) {
-              const bool kd = dropout_keeps(drop_col + (uint64_t)m * N, p.seed, p.dropout_p);
-              pd = kd ? pv : 0.f;
-              dpv = kd ? dp[r] * rp : 0.f;
+              pd = survivor(r, pv);
+              dpv = survivor(r, dp[r] * rp);
             }
             pr[r] = pd;
             ds[r] = FOLDED ? pv * (dpv + drow[r >> 2][r & 3]) : pv * (dpv - drow[r >> 2][r & 3]);
@@ -638,9 +663,8 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (DROP ? 1 : KvCfg<T, D, PW>::WAVES_PE
                                     : hw::exp2_fast(fmaf(s[r], c2, -lrow[r >> 2][r & 3]));
             float pd = pv, dpv = dp[r];
             if (DROP) {
-              const bool kd = dropout_keeps(drop_col + (uint64_t)(mr0 + block_row(r, hh)) * N, p.seed, p.dropout_p);
-              pd = kd ? pv : 0.f;
-              dpv = kd ? dp[r] * rp : 0.f;
+              pd = survivor(r, pv);
+              dpv = survivor(r, dp[r] * rp);
             }
             pr[r] = pd;
             ds[r] = FOLDED ? pv * (dpv + drow[r >> 2][r & 3]) : pv * (dpv - drow[r >> 2][r & 3]);
@@ -720,8 +744,9 @@ struct QCfg {
 
 // PW: two passes over the key tiles, as in the forward kernel -- the far keys with (q2, k2)
 // accumulating dQ2, then the near keys with (q1, k1) accumulating dQ1 in the same registers.
-// DROP: dP is masked and scaled by 1 / (1 - dropout_p) before dS = P (dP - delta) (flash.py:877-890).
-template <class T, int D, bool PW, bool DROP = false>
+// DROP: dP is masked and scaled by 1 / (1 - dropout_p) before dS = P (dP - delta) (flash.py:877-890); 1: the mask is
+// drawn again, 2: read as the forward left it, one word per lane and key block, a tile ahead.
+template <class T, int D, bool PW, int DROP = 0>
 FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_bwd_dq_kernel(BwdParams p) {
   static_assert(!(PW && DROP), "piecewise attention has no dropout");
   using C = QCfg<T, D, PW>;
@@ -758,7 +783,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
   const float d_row = my_m < M ? p.delta[row_off] : 0.f;
   const float rp = DROP ? 1.f / (1.f - p.dropout_p) : 1.f;
   // dropout counter of (my_m, key 0)
-  const uint64_t drop_row = DROP ? p.offset + (((uint64_t)batch * p.H + head) * M + (uint64_t)(my_m < M ? my_m : 0)) * N : 0;
+  const uint64_t drop_row = DROP == 1 ? p.offset + (((uint64_t)batch * p.H + head) * M + (uint64_t)(my_m < M ? my_m : 0)) * N : 0;
 
   int hi = N;
   if (p.causal) hi = imin(N, pseq + m0 + C::BM);
@@ -780,8 +805,12 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
   int64_t k_stride = 0;
   TileMover<T, C::BN, D> kr, vr;
   vr.init(tid, p.v.st);
+  const KeepMask keep_at(M, N);
+  const uint32_t* keep_lane = DROP == 2 ? p.keep + keep_at.head((int64_t)batch * p.H + head) + (my_m < keep_at.rows ? my_m : 0) : nullptr;
+  uint32_t keep_reg[2] = {0u, 0u};
   auto fetch = [&](int n0) {
     const int rows = N - n0;
+    if (DROP == 2) { keep_reg[0] = keep_lane[keep_at.block(n0 / 32)]; keep_reg[1] = keep_lane[keep_at.block(n0 / 32 + 1)]; }
     kr.fetch(k_src + (int64_t)n0 * k_stride, rows);
     vr.fetch(vb + (int64_t)n0 * p.v.st, rows);
   };
@@ -838,13 +867,14 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
     }
     hw::wait_global_loads();  // Q and dO rows
 
-    // One key tile.  `plain`: no mask touches the tile for any row of this wavefront (and there is no dropout or
+    // One key tile.  `plain`: no mask touches the tile for any row of this wavefront (and nothing is drawn and there is no
     // second regime), so the body has no branch and the compiler may run the element-wise work of one 32-key block
     // under the matrix instructions of the other.  The two variants run in loops of their own.
     auto tile = [&](auto plain_tag, int it) {
       constexpr bool plain = decltype(plain_tag)::value;
       const int n0 = it * C::BN;
       const bool more = it + 1 < t_end;
+      const uint32_t keep_word[2] = {keep_reg[0] >> (4 * hh), keep_reg[1] >> (4 * hh)};   // loaded ahead of the tile's rows
       if (more) fetch(n0 + C::BN);
 
       const T* sK = (const T*)(smem + stage * C::STAGE_BYTES);
@@ -871,6 +901,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
         bool need_mask = !plain && ((nlo + 32 > N) || (p.causal && (nlo + 31 > pseq + mw)));
         if (PW) need_mask = need_mask || (far_phase ? (mw + pseq - (nlo + 31) < p.w) : (mw + 31 + pseq - nlo >= p.w));
         f32x16 ds;
+        const uint32_t drawn = DROP == 1 ? dropout_draw16(drop_row + (uint64_t)(nlo + 4 * hh), p.seed, p.threshold) : 0u;
+        auto survivor = [&](int r, float x) {
+          return DROP == 2 ? hw::keep_if_bit(x, keep_word[nb], block_row(r, 0)) : hw::keep_if_bit(x, drawn, r);
+        };
         if (need_mask) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
@@ -880,15 +914,14 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
             float pv = hw::exp2_fast(fmaf(s[r], c2, -l_row));
             pv = keep ? pv : 0.f;
             float dpv = dp[r];
-            if (DROP) dpv = dropout_keeps(drop_row + (uint64_t)n, p.seed, p.dropout_p) ? dp[r] * rp : 0.f;
+            if (DROP) dpv = survivor(r, dp[r] * rp);
             ds[r] = pv * (dpv - d_row);
           }
         } else {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             float dpv = dp[r];
-            if (DROP)
-              dpv = dropout_keeps(drop_row + (uint64_t)(nlo + block_row(r, hh)), p.seed, p.dropout_p) ? dp[r] * rp : 0.f;
+            if (DROP) dpv = survivor(r, dp[r] * rp);
             ds[r] = hw::exp2_fast(fmaf(s[r], c2, -l_row)) * (dpv - d_row);
           }
         }
@@ -907,7 +940,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
     };
     {
       int it = t_begin;
-      if constexpr (!PW && !DROP) {
+      if constexpr (!PW && DROP != 1) {
         // tiles whose 64 keys exist and are visible to the wavefront's first row
         int plain_end = imin(t_end, N / C::BN);
         if (p.causal) plain_end = imin(plain_end, imax(0, mw + pseq + 1) / C::BN);
@@ -1086,20 +1119,20 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_bwd_dq_from_ds_kernel(BwdParams
 }
 
 // ------------------------------------------------------------------------------ launchers ----
-template <class T, bool PW, bool DS, bool DROP, bool GROUPED>
+template <class T, bool PW, bool DS, int DROP, bool GROUPED>
 static int launch_dkdv(const BwdParams& p, hipStream_t stream) {
   const int chunk = GROUPED ? (p.chunk > 0 ? p.chunk : p.group) : 1;
   dim3 grid(((p.N + 127) / 128) * (p.H / chunk) * p.B, 1, 1);
   switch (p.D) {
-    case 16: return launch(fa_bwd_dkdv_kernel<T, 16, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 16, PW>::LDS_BYTES, stream, p);
-    case 32: return launch(fa_bwd_dkdv_kernel<T, 32, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 32, PW>::LDS_BYTES, stream, p);
-    case 64: return launch(fa_bwd_dkdv_kernel<T, 64, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 64, PW>::LDS_BYTES, stream, p);
-    case 128: return launch(fa_bwd_dkdv_kernel<T, 128, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 128, PW>::LDS_BYTES, stream, p);
+    case 16: return launch(fa_bwd_dkdv_kernel<T, 16, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 16, PW, DROP>::LDS_BYTES, stream, p);
+    case 32: return launch(fa_bwd_dkdv_kernel<T, 32, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 32, PW, DROP>::LDS_BYTES, stream, p);
+    case 64: return launch(fa_bwd_dkdv_kernel<T, 64, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 64, PW, DROP>::LDS_BYTES, stream, p);
+    case 128: return launch(fa_bwd_dkdv_kernel<T, 128, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 128, PW, DROP>::LDS_BYTES, stream, p);
   }
   return kUnsupported;
 }
 
-template <class T, bool PW, bool DROP>
+template <class T, bool PW, int DROP>
 static int launch_dq(const BwdParams& p, hipStream_t stream) {
   dim3 grid(((p.M + 127) / 128) * p.H * p.B, 1, 1);
   switch (p.D) {
@@ -1126,32 +1159,40 @@ static bool dkdv_chunk_ok(const BwdParams& p, bool piecewise) {
 
 template <class T>
 static int dispatch_dkdv(const BwdParams& p, bool piecewise, bool keep_ds, hipStream_t stream) {
-  if (piecewise) return keep_ds ? launch_dkdv<T, true, true, false, false>(p, stream) : launch_dkdv<T, true, false, false, false>(p, stream);
+  if (piecewise) return keep_ds ? launch_dkdv<T, true, true, 0, false>(p, stream) : launch_dkdv<T, true, false, 0, false>(p, stream);
   const bool drop = p.dropout_p > 0.f;
   const bool grouped = (p.chunk > 0 ? p.chunk : p.group) > 1;
   if (keep_ds) {
-    if (drop) return launch_dkdv<T, false, true, true, false>(p, stream);
-    return grouped ? launch_dkdv<T, false, true, false, true>(p, stream) : launch_dkdv<T, false, true, false, false>(p, stream);
+    if (drop) return p.keep ? launch_dkdv<T, false, true, 2, false>(p, stream) : launch_dkdv<T, false, true, 1, false>(p, stream);
+    return grouped ? launch_dkdv<T, false, true, 0, true>(p, stream) : launch_dkdv<T, false, true, 0, false>(p, stream);
   }
-  if (drop) return launch_dkdv<T, false, false, true, false>(p, stream);
-  return grouped ? launch_dkdv<T, false, false, false, true>(p, stream) : launch_dkdv<T, false, false, false, false>(p, stream);
+  if (drop) return p.keep ? launch_dkdv<T, false, false, 2, false>(p, stream) : launch_dkdv<T, false, false, 1, false>(p, stream);
+  return grouped ? launch_dkdv<T, false, false, 0, true>(p, stream) : launch_dkdv<T, false, false, 0, false>(p, stream);
 }
 
 template <class T>
 static int dispatch_dq(const BwdParams& p, bool piecewise, hipStream_t stream) {
-  if (piecewise) return launch_dq<T, true, false>(p, stream);
-  return p.dropout_p > 0.f ? launch_dq<T, false, true>(p, stream) : launch_dq<T, false, false>(p, stream);
+  if (piecewise) return launch_dq<T, true, 0>(p, stream);
+  if (p.dropout_p > 0.f) return p.keep ? launch_dq<T, false, 2>(p, stream) : launch_dq<T, false, 1>(p, stream);
+  return launch_dq<T, false, 0>(p, stream);
 }
 
-int run_bwd_dkdv(const BwdParams& p, bool piecewise, hipStream_t stream) {
-  if (!bwd_args_ok(p, piecewise) || !dkdv_chunk_ok(p, piecewise)) return kBadArgument;
+static BwdParams with_threshold(BwdParams p) {
+  p.threshold = p.dropout_p > 0.f ? dropout_threshold(p.dropout_p) : 0u;
+  return p;
+}
+
+int run_bwd_dkdv(const BwdParams& a, bool piecewise, hipStream_t stream) {
+  if (!bwd_args_ok(a, piecewise) || !dkdv_chunk_ok(a, piecewise)) return kBadArgument;
+  const BwdParams p = with_threshold(a);
   if (p.dtype == kDtypeF16) return dispatch_dkdv<hw::half_t>(p, piecewise, false, stream);
   if (p.dtype == kDtypeBF16) return dispatch_dkdv<hw::bf16_t>(p, piecewise, false, stream);
   return kUnsupported;
 }
 
-int run_bwd_dq(const BwdParams& p, bool piecewise, hipStream_t stream) {
-  if (!bwd_args_ok(p, piecewise)) return kBadArgument;
+int run_bwd_dq(const BwdParams& a, bool piecewise, hipStream_t stream) {
+  if (!bwd_args_ok(a, piecewise)) return kBadArgument;
+  const BwdParams p = with_threshold(a);
   if (p.dtype == kDtypeF16) return dispatch_dq<hw::half_t>(p, piecewise, stream);
   if (p.dtype == kDtypeBF16) return dispatch_dq<hw::bf16_t>(p, piecewise, stream);
   return kUnsupported;
@@ -1173,8 +1214,9 @@ int64_t bwd_ds_workspace_bytes(int B, int H, int M, int N) {
   return (int64_t)B * H * (4 * (int64_t)((M + 127) / 128)) * (4 * (int64_t)((N + 127) / 128)) * 2048;
 }
 
-int run_bwd_dkdv_ds(const BwdParams& p, bool piecewise, hipStream_t stream) {
-  if (!bwd_args_ok(p, piecewise) || !dkdv_chunk_ok(p, piecewise) || !p.ds) return kBadArgument;
+int run_bwd_dkdv_ds(const BwdParams& a, bool piecewise, hipStream_t stream) {
+  if (!bwd_args_ok(a, piecewise) || !dkdv_chunk_ok(a, piecewise) || !a.ds) return kBadArgument;
+  const BwdParams p = with_threshold(a);
   if (p.dtype == kDtypeF16) return dispatch_dkdv<hw::half_t>(p, piecewise, true, stream);
   if (p.dtype == kDtypeBF16) return dispatch_dkdv<hw::bf16_t>(p, piecewise, true, stream);
   return kUnsupported;

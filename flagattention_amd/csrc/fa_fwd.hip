@@ -82,7 +82,9 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
   const float c2 = p.sm_scale * kLog2e;
   constexpr float kLazyBits = 8.f;
   const float lazy_tau = c2 > 0.f ? kLazyBits / c2 : 0.f;   // in units of raw scores; a non-positive scale keeps the exact maximum
-  // dropout counter of (my_m, key 0)
+  // dropout counter of (my_m, key 0), and where this row's words of the mask go
+  const KeepMask keep_at(M, N);
+  uint32_t* const keep_row = DROP && p.keep && mw < M ? p.keep + keep_at.head((int64_t)batch * p.H + head) + my_m : nullptr;
   const uint64_t drop_row = DROP ? p.offset + (((uint64_t)batch * p.H + head) * M + (uint64_t)(my_m < M ? my_m : 0)) * N : 0;
   float m_i = neg_inf(), l_i = 0.f;
   f32x16 oacc[C::DV / 32];
@@ -172,13 +174,24 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
     const float m_use = (m_new == neg_inf()) ? 0.f : m_new;  // row with no visible key so far
     const float shift = -m_use * c2;
     float psum = 0.f;
+    uint32_t keep_bits[C::BN / 32];
+    if (DROP) {
+#pragma unroll
+      for (int nb = 0; nb < C::BN / 32; ++nb)
+        keep_bits[nb] = dropout_draw16(drop_row + (uint64_t)(n0 + nb * 32 + 4 * hh), p.seed, p.threshold);
+      if (p.keep) {   // a lane and its lane^32 twin hold the two halves of a row's words; each stores one of them
+        const uint32_t mine0 = keep_spread(keep_bits[0], hh), mine1 = keep_spread(keep_bits[1], hh);
+        const float other = hw::xor32(__builtin_bit_cast(float, hh ? mine0 : mine1));
+        if (keep_row) keep_row[keep_at.block(n0 / 32 + hh)] = (hh ? mine1 : mine0) | __builtin_bit_cast(uint32_t, other);
+      }
+    }
 #pragma unroll
     for (int nb = 0; nb < C::BN / 32; ++nb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         float e = hw::exp2_fast(fmaf(s[nb][r], c2, shift));
         psum += e;
-        if (DROP) e = dropout_keeps(drop_row + (uint64_t)(n0 + nb * 32 + block_row(r, hh)), p.seed, p.dropout_p) ? e : 0.f;
+        if (DROP) e = hw::keep_if_bit(e, keep_bits[nb], r);
         s[nb][r] = e;
       }
     // The accumulators are rescaled only when some row of the wavefront raised its maximum;
@@ -306,8 +319,10 @@ int run_fwd(const FwdParams& p, bool piecewise, hipStream_t stream) {
   if (p.block_m != 0 && p.block_m != 128 && p.block_m != 256) return kUnsupported;
   if (p.block_m == 256 && (piecewise || !fwd_wide_supported(p))) return kUnsupported;
   if (!piecewise && (p.block_m == 256 || (p.block_m == 0 && fwd_wide_supported(p) && prefer_wide(p)))) return run_fwd_wide(p, stream);
-  if (p.dtype == kDtypeF16) return dispatch_fwd<hw::half_t>(p, piecewise, stream);
-  if (p.dtype == kDtypeBF16) return dispatch_fwd<hw::bf16_t>(p, piecewise, stream);
+  FwdParams d = p;
+  d.threshold = p.dropout_p > 0.f ? dropout_threshold(p.dropout_p) : 0u;
+  if (p.dtype == kDtypeF16) return dispatch_fwd<hw::half_t>(d, piecewise, stream);
+  if (p.dtype == kDtypeBF16) return dispatch_fwd<hw::bf16_t>(d, piecewise, stream);
   return kUnsupported;
 }
 

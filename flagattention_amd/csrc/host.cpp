@@ -217,8 +217,13 @@ bool plan_flash(FlashPlan& plan, int64_t B, int64_t H, int64_t Hk, int64_t M, in
   return true;
 }
 
-// o, L and (if asked for) the column sums
-variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, const FlashCall& c, const FlashPlan& plan) {
+// The mask goes to the backward as bits where they take at most as much memory as q, k, v and o do, which are kept
+// too: N / 8 bytes per query row against 8 D (equal heads).  Beyond that the backward draws it again.
+bool keeps_mask(int64_t N, int64_t D) { return N <= 64 * D; }
+
+// o, L and (if asked for) the column sums; with dropout, the mask for a backward if `keep` is given
+variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, const FlashCall& c, const FlashPlan& plan,
+                            Tensor* keep = nullptr) {
   const int B = (int)q.size(0), H = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3);
   const int Hk = (int)k.size(1), N = (int)k.size(2), type = dtype_code(q);
   void* stream = stream_of(q);
@@ -243,8 +248,14 @@ variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, c
     o = empty_result(q);
     L = empty({B, H, M}, at::kFloat, q);
     const fa_view4 vo = view4(o);
-    check(fa_fwd(type, &vq, &vk, &vv, &vo, f32(L), B, H, Hk, M, N, D, c.causal, (float)c.scale, (float)c.dropout_p,
-                 c.seed, c.offset, 0, stream), "fa_fwd");
+    if (keep && c.dropout_p > 0 && keeps_mask(N, D)) {
+      *keep = empty({(int64_t)B * H * fa_dropout_keep_words(M, N)}, at::kInt, q);
+      check(fa_fwd_keep(type, &vq, &vk, &vv, &vo, f32(L), (uint32_t*)keep->mutable_data_ptr(), B, H, Hk, M, N, D, c.causal,
+                        (float)c.scale, (float)c.dropout_p, c.seed, c.offset, stream), "fa_fwd_keep");
+    } else {
+      check(fa_fwd(type, &vq, &vk, &vv, &vo, f32(L), B, H, Hk, M, N, D, c.causal, (float)c.scale, (float)c.dropout_p,
+                   c.seed, c.offset, 0, stream), "fa_fwd");
+    }
   }
   variable_list out = {o, L};
   if (c.want_total) {
@@ -257,7 +268,7 @@ variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, c
 }
 
 variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& L,
-                             const Tensor& grad, const FlashCall& c, int64_t limit_mib) {
+                             const Tensor& keep, const Tensor& grad, const FlashCall& c, int64_t limit_mib) {
   const int B = (int)q.size(0), H = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3);
   const int Hk = (int)k.size(1), N = (int)k.size(2), group = H / Hk, type = dtype_code(q);
   const Tensor g = kernel_ready(grad);
@@ -276,14 +287,24 @@ variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, 
   Tensor ds;
   if (heads >= (int64_t)B * H) ds = ds_workspace(q, B, H, M, N, 1);
   else if (heads > 0) ds = ds_workspace(q, 1, heads = std::min<int64_t>(heads, H), M, N, 1);
-  if (!ds.defined()) {   // dS not worth keeping for this shape, or no memory for it: recompute it
+  const uint32_t* bits = keep.defined() ? (const uint32_t*)keep.const_data_ptr() : nullptr;
+  if (!ds.defined() && bits) {
+    check(fa_bwd_dkdv_keep(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, nullptr, 0, bits, B, H, Hk, M, N, D,
+                           c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
+    check(fa_bwd_dq_keep(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdq, bits, B, H, Hk, M, N, D, c.causal, scale, p,
+                         stream), "fa_bwd_dq_keep");
+  } else if (!ds.defined()) {   // dS not worth keeping for this shape, or no memory for it: recompute it
     check(fa_bwd_dkdv(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, B, H, Hk, M, N, D, c.causal,
                       scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv");
     check(fa_bwd_dq(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdq, B, H, Hk, M, N, D, c.causal, scale, p, c.seed,
                     c.offset, stream), "fa_bwd_dq");
   } else if (heads >= (int64_t)B * H) {
-    check(fa_bwd_dkdv_ds(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, ds.mutable_data_ptr(),
-                         ds.numel(), B, H, Hk, M, N, D, c.causal, scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv_ds");
+    if (bits)
+      check(fa_bwd_dkdv_keep(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, ds.mutable_data_ptr(), ds.numel(),
+                             bits, B, H, Hk, M, N, D, c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
+    else
+      check(fa_bwd_dkdv_ds(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, ds.mutable_data_ptr(),
+                           ds.numel(), B, H, Hk, M, N, D, c.causal, scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv_ds");
     check(fa_bwd_dq_from_ds(type, &vk, ds.const_data_ptr(), ds.numel(), &vdq, B, H, Hk, M, N, D, c.causal, scale,
                             stream), "fa_bwd_dq_from_ds");
   } else {
@@ -296,9 +317,14 @@ variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, 
                        sg = slice4(g, b, h0), sdk = slice4(dk, b, h0 / chunk), sdv = slice4(dv, b, h0 / chunk),
                        sdq = slice4(dq, b, h0);
         const int64_t row = (b * H + h0) * M;
-        check(fa_bwd_dkdv_ds(type, &sq, &sk, &sv, &sg, f32(L) + row, f32(delta) + row, &sdk, &sdv, chunk,
-                             ds.mutable_data_ptr(), ds.numel(), 1, n, kn, M, N, D, c.causal, scale, p, c.seed,
-                             c.offset + (uint64_t)row * (uint64_t)N, stream), "fa_bwd_dkdv_ds");
+        if (bits)
+          check(fa_bwd_dkdv_keep(type, &sq, &sk, &sv, &sg, f32(L) + row, f32(delta) + row, &sdk, &sdv, ds.mutable_data_ptr(),
+                                 ds.numel(), bits + (b * H + h0) * fa_dropout_keep_words(M, N), 1, n, kn, M, N, D,
+                                 c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
+        else
+          check(fa_bwd_dkdv_ds(type, &sq, &sk, &sv, &sg, f32(L) + row, f32(delta) + row, &sdk, &sdv, chunk,
+                               ds.mutable_data_ptr(), ds.numel(), 1, n, kn, M, N, D, c.causal, scale, p, c.seed,
+                               c.offset + (uint64_t)row * (uint64_t)N, stream), "fa_bwd_dkdv_ds");
         check(fa_bwd_dq_from_ds(type, &sk, ds.const_data_ptr(), ds.numel(), &sdq, 1, n, kn, M, N, D, c.causal, scale,
                                 stream), "fa_bwd_dq_from_ds");
       }
@@ -317,8 +343,11 @@ struct Held : torch::CustomClassHolder {   // a call's parameters as one saved v
 };
 template <class Call>
 void hold(AutogradContext* ctx, const Call& c) {
+  ctx->set_materialize_grads(false);   // no zeroes for the outputs whose gradients are ignored
   ctx->saved_data["call"] = c10::IValue::make_capsule(c10::make_intrusive<Held<Call>>(c));
 }
+// the gradient of the output o: zero where nothing flows into it
+Tensor gradient_of(const Tensor& o, const Tensor& grad) { return grad.defined() ? grad : at::zeros_like(o); }
 template <class Call>
 const Call& held(AutogradContext* ctx) {
   return static_cast<Held<Call>*>(ctx->saved_data["call"].toCapsule().get())->call;
@@ -328,8 +357,9 @@ struct FlashNode : torch::autograd::Function<FlashNode> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q0, const Tensor& k0, const Tensor& v0,
                                const FlashCall& c, const FlashPlan& plan) {
     const Tensor q = kernel_ready(q0), k = kernel_ready(k0), v = kernel_ready(v0);
-    variable_list out = flash_forward(q, k, v, c, plan);
-    ctx->save_for_backward({q, k, v, out[0], out[1]});
+    Tensor keep;
+    variable_list out = flash_forward(q, k, v, c, plan, &keep);
+    ctx->save_for_backward({q, k, v, out[0], out[1], keep});
     hold(ctx, c);
     return out;
   }
@@ -339,7 +369,8 @@ struct FlashNode : torch::autograd::Function<FlashNode> {
     const Tensor &q = saved[0], &k = saved[1];
     const c10::DeviceGuard guard(q.device());
     const int64_t limit = backward_settings(g_flash_settings, q.size(0), q.size(1), q.size(2), k.size(2), q.size(3), c.causal);
-    variable_list r = flash_backward(q, k, saved[2], saved[3], saved[4], grads[0], c, limit);
+    variable_list r = flash_backward(q, k, saved[2], saved[3], saved[4], saved[5],
+                                     gradient_of(saved[3], grads[0]), c, limit);
     return {r[0], r[1], r[2], Tensor(), Tensor()};
   }
 };
@@ -444,7 +475,7 @@ struct PiecewiseNode : torch::autograd::Function<PiecewiseNode> {
     const int B = (int)q1.size(0), H = (int)q1.size(1), M = (int)q1.size(2), D = (int)q1.size(3), N = (int)k1.size(2);
     const c10::DeviceGuard guard(q1.device());
     const int64_t limit = backward_settings(g_piecewise_settings, B, H, M, N, D, c.causal);
-    const Tensor g = kernel_ready(grads[0]);
+    const Tensor g = kernel_ready(gradient_of(o, grads[0]));
     const int type = dtype_code(q1);
     const float scale = (float)c.scale;
     void* stream = stream_of(q1);

@@ -163,6 +163,17 @@ FA_DEVICE void swap_halves(float& a, float& b) {
 // either side of it.
 FA_DEVICE void swap_halves_in_slot(float& a, float& b) { asm volatile("v_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
 
+// a ^ b ^ c in one instruction.
+FA_DEVICE uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96); }
+// bits = 2 bits + (x >= bound): the comparison's carry goes straight into the addition.
+FA_DEVICE void append_at_least(uint32_t& bits, uint32_t x, uint32_t bound) {
+  asm("v_cmp_ge_u32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(bits) : "v"(x), "s"(bound) : "vcc");
+}
+// x where bit `pos` of `bits` is set, else 0 (a mask, so that no arithmetic touches x).
+FA_DEVICE float keep_if_bit(float x, uint32_t bits, int pos) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & (uint32_t)__builtin_amdgcn_sbfe((int)bits, (uint32_t)pos, 1u));
+}
+
 // Tells the compiler that x has the same value in every lane (kept in a scalar register).
 FA_DEVICE int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 

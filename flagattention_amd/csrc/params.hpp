@@ -22,7 +22,9 @@ struct FwdParams {
   float sm_scale;
   int dtype;
   float dropout_p;        // 0 = no dropout; otherwise the mask is drawn from (seed, offset)
+  uint32_t threshold;     // dropout_threshold(dropout_p), filled in by run_fwd
   uint64_t seed, offset;
+  uint32_t* keep;         // optional: the drawn mask for the backward (KeepMask in common.hpp)
   int block_m;            // query rows per workgroup: 128, 256, or 0 = the library's choice
   // 256-row kernel over pieces of the key axis (0 = the whole axis, results to o / lse): piece s covers keys
   // s * split_size .. + split_size - 1 and leaves its normalised output as fp16 in part_o (B, H, num_splits, M, D)
@@ -48,7 +50,9 @@ struct BwdParams {
   float sm_scale;
   int dtype;
   float dropout_p;
+  uint32_t threshold;     // dropout_threshold(dropout_p), filled in by the launchers
   uint64_t seed, offset;
+  const uint32_t* keep;   // the forward's mask, or null: drawn again from (seed, offset)
 };
 
 struct TotalParams {
@@ -124,6 +128,7 @@ struct MaskParams {
   uint8_t* mask;   // (B, H, M, N) contiguous, one byte per element: 1 = kept
   int64_t total;   // B * H * M * N
   float dropout_p;
+  uint32_t threshold;   // filled in by run_dropout_mask
   uint64_t seed, offset;
 };
 int run_dropout_mask(const MaskParams& p, hipStream_t stream);
@@ -138,6 +143,7 @@ struct ProbeParams {
 };
 int run_probe_mfma(const ProbeParams& p, hipStream_t stream);
 
+inline int64_t dropout_keep_words(int M, int N) { return 64 * (int64_t)((M + 31) / 32) * ((N + 63) / 64); }   // per (batch, head)
 int64_t bwd_ds_workspace_bytes(int B, int H, int M, int N);
 int run_bwd_dkdv_ds(const BwdParams& p, bool piecewise, hipStream_t stream);
 int run_bwd_dq_from_ds(const BwdParams& p, bool piecewise, hipStream_t stream);

@@ -70,6 +70,15 @@ int fa_fwd(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, c
            float* lse, int B, int H, int Hk, int M, int N, int D, int causal, float sm_scale,
            float dropout_p, uint64_t seed, uint64_t offset, int block_m, void* stream);
 
+/* The same with dropout whose mask is kept for the backward (no counterpart in the reference, whose backward kernels
+ * draw it again, flash.py:697-721, 877-890: drawing is two to three times the work of the rest of a kernel).
+ * dropout_p > 0.  keep: B * H * fa_dropout_keep_words(M, N) 32-bit words (one bit per score), 4-byte aligned, in a private
+ * order; its contents on entry do not matter. */
+int fa_dropout_keep_words(int M, int N);
+int fa_fwd_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* o, float* lse,
+                uint32_t* keep, int B, int H, int Hk, int M, int N, int D, int causal, float sm_scale, float dropout_p,
+                uint64_t seed, uint64_t offset, void* stream);
+
 /* ----------------------------------------------------------------- flash attention, backward --
  * The reference's three launches in FlashAttention.backward, src/flag_attn/flash.py:191-249:
  *
@@ -115,6 +124,16 @@ int fa_bwd_dkdv_ds(int dtype, const fa_view4* q, const fa_view4* k, const fa_vie
 int fa_bwd_dq_from_ds(int dtype, const fa_view4* k, const void* ds_workspace, int64_t ds_workspace_bytes,
                       const fa_view4* dq, int B, int H, int Hk, int M, int N, int D, int causal,
                       float sm_scale, void* stream);
+
+/* fa_bwd_dkdv / fa_bwd_dkdv_ds (with a workspace; null and 0 bytes without) and fa_bwd_dq with the mask that
+ * fa_fwd_keep left: same B, H, M, N, causal flag and dropout_p, one dK / dV slice per query head. */
+int fa_bwd_dkdv_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* dout,
+                     const float* lse, const float* delta, const fa_view4* dk, const fa_view4* dv, void* ds_workspace,
+                     int64_t ds_workspace_bytes, const uint32_t* keep, int B, int H, int Hk, int M, int N, int D,
+                     int causal, float sm_scale, float dropout_p, void* stream);
+int fa_bwd_dq_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* dout,
+                   const float* lse, const float* delta, const fa_view4* dq, const uint32_t* keep, int B, int H, int Hk,
+                   int M, int N, int D, int causal, float sm_scale, float dropout_p, void* stream);
 
 /* ------------------------------------------------------------------------- total attention --
  * Replaces `_total_attention_kernel` (src/flag_attn/total.py:50-142; launches flash.py:128-140 and

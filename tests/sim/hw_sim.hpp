@@ -342,6 +342,9 @@ inline int lane_value(int x, int lane) {
   }
   return result;
 }
+inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return a ^ b ^ c; }
+inline void append_at_least(uint32_t& bits, uint32_t x, uint32_t bound) { bits = 2 * bits + (x >= bound ? 1u : 0u); }
+inline float keep_if_bit(float x, uint32_t bits, int pos) { return (bits >> pos) & 1u ? x : 0.f; }
 inline int read_lane(int x, int lane) {   // in halves: lane_value() passes through a float
   return (int)((uint32_t)lane_value((int)((uint32_t)x >> 16), lane) << 16 | (uint32_t)lane_value(x & 0xffff, lane));
 }

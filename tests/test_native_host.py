@@ -81,6 +81,31 @@ def test_native_dropout_draws_like_the_python_path():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,H,Hk,M,N,D,causal", [
+    (8, 16, 16, 129, 129, 64, True),       # rows and keys one past a tile
+    (8, 16, 8, 31, 97, 16, False),         # less than a block of rows, three blocks of keys
+    (4, 32, 32, 160, 33, 32, True),        # rows that see no key
+    (16, 16, 16, 100, 64, 128, False),
+    (4, 16, 4, 1100, 1030, 128, True),     # dS kept
+])
+def test_kept_dropout_mask_gives_the_gradients_of_a_drawn_one(B, H, Hk, M, N, D, causal):
+    """The native path hands the forward's mask to the backward as bits, the Python path draws it again: the same
+    elements survive, so all results are equal bit for bit -- with a counter whose upper word changes inside the call."""
+    q, k, v = (randn(B, h, t, D, grad=True) for h, t in ((H, M), (Hk, N), (Hk, N)))
+    do = randn(B, H, M, D)
+    gen = torch.cuda.default_generators[0]
+    results = []
+    for call in (flag_attn.flash_attention, flash.FlashAttention.apply):
+        gen.manual_seed(2 ** 40 + 3)
+        gen.set_offset(2 ** 32 - 4 * (B * H * M * N // 8))
+        o, _, _, seed, offset = call(q, k, v, causal, None, 0.3, False, False, True)
+        assert offset < 2 ** 32 < offset + B * H * M * N
+        results.append((o,) + torch.autograd.grad(o, (q, k, v), do))
+    for name, a, b in zip(("o", "dq", "dk", "dv"), *results):
+        assert torch.equal(a, b), name
+
+
+@pytest.mark.gpu
 def test_calls_the_native_path_does_not_take_still_raise():
     q, k = randn(1, 4, 64, 64), randn(1, 3, 64, 64)
     with pytest.raises(AssertionError):
