@@ -129,44 +129,61 @@ def fa_bwd_delta(lib, o, do, delta):
           "fa_bwd_delta")
 
 
-def _heads_per_slice(q, dk):
-    """dk / dv hold one slice per this many query heads (summed by the kernel)."""
-    H, slices = q.shape[1], dk.shape[1]
+def _heads_per_slice(q, dk, pieces=1):
+    """dk / dv hold one slice per this many query heads (summed by the kernel) and piece."""
+    H, slices = q.shape[1], dk.shape[1] // max(1, pieces)
     assert H % slices == 0
     return H // slices
 
 
-def fa_bwd_dkdv(lib, q, k, v, do, lse, delta, dk, dv, causal, sm_scale, dropout=NO_DROPOUT):
+def pieces_code(pieces):
+    """FA_PIECES of include/flagattn.h: added to a dtype code, results as that many fp32 slices (0: results as they are)."""
+    return pieces << 8
+
+
+def fa_sum_slices(lib, slices, outs):
+    """outs[t] = slices[t].sum(dim) over the one dimension that slices[t] (fp32) has more, for up to three tensors."""
+    n = len(outs)
+    counts = [s.numel() // o.numel() for s, o in zip(slices, outs)]
+    inner = [o.shape[-1] * o.shape[-2] for o in outs]
+    pointers, longs, ints = ctypes.c_void_p * n, ctypes.c_int64 * n, ctypes.c_int32 * n
+    check(lib.fa_sum_slices(dtype_code(outs[0]), pointers(*(s.data_ptr() for s in slices)), pointers(*(o.data_ptr() for o in outs)),
+                            longs(*(o.numel() // i for o, i in zip(outs, inner))), ints(*counts), longs(*inner), n,
+                            stream_of(outs[0])), "fa_sum_slices")
+
+
+def fa_bwd_dkdv(lib, q, k, v, do, lse, delta, dk, dv, causal, sm_scale, dropout=NO_DROPOUT, pieces=0):
     B, H, M, D = q.shape
     Hk, N = k.shape[1], k.shape[2]
-    check(lib.fa_bwd_dkdv(dtype_code(q), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta),
-                          view4(dk), view4(dv), _heads_per_slice(q, dk), B, H, Hk, M, N, D, int(causal),
+    check(lib.fa_bwd_dkdv(dtype_code(q) | pieces_code(pieces), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta),
+                          view4(dk), view4(dv), _heads_per_slice(q, dk, pieces), B, H, Hk, M, N, D, int(causal),
                           float(sm_scale), float(dropout[0]), _u64(dropout[1]), _u64(dropout[2]),
                           stream_of(q)), "fa_bwd_dkdv")
 
 
-def fa_bwd_dq(lib, q, k, v, do, lse, delta, dq, causal, sm_scale, dropout=NO_DROPOUT):
+def fa_bwd_dq(lib, q, k, v, do, lse, delta, dq, causal, sm_scale, dropout=NO_DROPOUT, pieces=0):
     B, H, M, D = q.shape
     Hk, N = k.shape[1], k.shape[2]
-    check(lib.fa_bwd_dq(dtype_code(q), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta),
+    check(lib.fa_bwd_dq(dtype_code(q) | pieces_code(pieces), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta),
                         view4(dq), B, H, Hk, M, N, D, int(causal), float(sm_scale), float(dropout[0]),
                         _u64(dropout[1]), _u64(dropout[2]), stream_of(q)), "fa_bwd_dq")
 
 
-def fa_bwd_dkdv_ds(lib, q, k, v, do, lse, delta, dk, dv, ds, causal, sm_scale, dropout=NO_DROPOUT):
+def fa_bwd_dkdv_ds(lib, q, k, v, do, lse, delta, dk, dv, ds, causal, sm_scale, dropout=NO_DROPOUT, pieces=0):
     B, H, M, D = q.shape
     Hk, N = k.shape[1], k.shape[2]
-    check(lib.fa_bwd_dkdv_ds(dtype_code(q), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta),
-                             view4(dk), view4(dv), _heads_per_slice(q, dk), ptr(ds),
+    check(lib.fa_bwd_dkdv_ds(dtype_code(q) | pieces_code(pieces), view4(q), view4(k), view4(v), view4(do), ptr(lse), ptr(delta),
+                             view4(dk), view4(dv), _heads_per_slice(q, dk, pieces), ptr(ds),
                              ds.numel() * ds.element_size(), B, H, Hk, M, N, D, int(causal),
                              float(sm_scale), float(dropout[0]), _u64(dropout[1]), _u64(dropout[2]),
                              stream_of(q)), "fa_bwd_dkdv_ds")
 
 
-def fa_bwd_dq_from_ds(lib, k, ds, dq, causal, sm_scale):
+def fa_bwd_dq_from_ds(lib, k, ds, dq, causal, sm_scale, pieces=0):
     B, H, M, D = dq.shape
+    H //= max(1, pieces)
     Hk, N = k.shape[1], k.shape[2]
-    check(lib.fa_bwd_dq_from_ds(dtype_code(dq), view4(k), ptr(ds), ds.numel() * ds.element_size(),
+    check(lib.fa_bwd_dq_from_ds(dtype_code(k) | pieces_code(pieces), view4(k), ptr(ds), ds.numel() * ds.element_size(),
                                 view4(dq), B, H, Hk, M, N, D, int(causal), float(sm_scale),
                                 stream_of(dq)), "fa_bwd_dq_from_ds")
 

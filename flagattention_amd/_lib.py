@@ -28,6 +28,7 @@ SIGNATURES = {
     "fa_fwd_keep": [_i, _v, _v, _v, _v, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _f, _u64, _u64, _p],
     "fa_bwd_dkdv_keep": [_i, _v, _v, _v, _v, _p, _p, _v, _v, _p, _i64, _p, _i, _i, _i, _i, _i, _i, _i, _f, _f, _p],
     "fa_bwd_dq_keep": [_i, _v, _v, _v, _v, _p, _p, _v, _p, _i, _i, _i, _i, _i, _i, _i, _f, _f, _p],
+    "fa_sum_slices": [_i, _p, _p, _p, _p, _p, _i, _p],
     "fa_bwd_delta": [_i, _v, _v, _p, _i, _i, _i, _i, _p],
     "fa_bwd_dkdv": [_i, _v, _v, _v, _v, _p, _p, _v, _v, _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _u64, _u64, _p],
     "fa_bwd_dq": [_i, _v, _v, _v, _v, _p, _p, _v, _i, _i, _i, _i, _i, _i, _i, _f, _f, _u64, _u64, _p],

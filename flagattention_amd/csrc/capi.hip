@@ -133,7 +133,8 @@ static int fill_bwd(fa::BwdParams& p, int dtype, const fa_view4* q, const fa_vie
   p.q = to_view(q); p.k = to_view(k); p.v = to_view(v); p.dout = to_view(dout);
   p.lse = lse; p.delta = const_cast<float*>(delta);
   p.B = B; p.H = H; p.M = M; p.N = N; p.D = D;
-  p.group = H / Hk; p.causal = causal; p.sm_scale = sm_scale; p.dtype = dtype;
+  p.group = H / Hk; p.causal = causal; p.sm_scale = sm_scale;
+  p.dtype = dtype & 0xff; p.pieces = dtype >> 8;   // FA_PIECES
   return 0;
 }
 
@@ -191,6 +192,18 @@ int fa_bwd_dq_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_vie
   return fa::run_bwd_dq(p, false, (hipStream_t)stream);
 }
 
+int fa_sum_slices(int dtype, const float* const* slices, void* const* out, const int64_t* outer, const int32_t* count,
+                  const int64_t* inner, int tensors, void* stream) {
+  if (!slices || !out || !outer || !count || !inner || tensors <= 0 || tensors > 3) return FA_ERR_BAD_ARGUMENT;
+  fa::SumParams p = {};
+  for (int i = 0; i < tensors; ++i) {
+    p.item[i].slices = slices[i]; p.item[i].out = out[i];
+    p.item[i].outer = outer[i]; p.item[i].count = count[i]; p.item[i].inner = inner[i];
+  }
+  p.items = tensors; p.dtype = dtype;
+  return fa::run_sum_slices(p, (hipStream_t)stream);
+}
+
 int fa_bwd_ds_workspace_mib(int B, int H, int M, int N) {
   if (B <= 0 || H <= 0 || M <= 0 || N <= 0) return FA_ERR_BAD_ARGUMENT;
   const int64_t mib = (fa::bwd_ds_workspace_bytes(B, H, M, N) + (1 << 20) - 1) >> 20;
@@ -229,7 +242,8 @@ int fa_bwd_dq_from_ds(int dtype, const fa_view4* k, const void* ds_workspace, in
   p.k = to_view(k); p.dq = to_view(dq);
   p.ds = const_cast<void*>(ds_workspace);
   p.B = B; p.H = H; p.M = M; p.N = N; p.D = D; p.group = H / Hk;
-  p.causal = causal; p.sm_scale = sm_scale; p.dtype = dtype;
+  p.causal = causal; p.sm_scale = sm_scale;
+  p.dtype = dtype & 0xff; p.pieces = dtype >> 8;   // FA_PIECES
   return fa::run_bwd_dq_from_ds(p, false, (hipStream_t)stream);
 }
 

@@ -105,6 +105,11 @@ struct KvCfg {
 // again; 2: it is read as the forward left it (p.keep; B=4 H=16 T=1024 D=64 causal: 84 -> 42 us), every wavefront's
 // 64 words of a tile by way of LDS.
 //
+// Pieces (p.pieces > 0, plain attention): the query tiles of a key block are dealt to that many workgroups and every
+// workgroup leaves its sums in fp32, one slice of p.dk / p.dv per (chunk of heads, piece), which fa_sum_slices_kernel
+// adds.  For launches with fewer workgroups than the device holds, whose time is the longest workgroup's, and (one
+// piece) for several chunks per kv head: B=2 H=4 T=3950 D=64 causal (248 workgroups of up to 62 tiles): 69 -> 49 us.
+//
 // GROUPED: the workgroup walks more than one query head (see below); a separate instantiation,
 // because the extra loop level costs the single-head kernel 10 % through register allocation alone.
 template <class T, int D, bool PW, bool DS = false, int DROP = 0, bool GROUPED = false>
@@ -122,13 +127,15 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (KvCfg<T, D, PW, DROP>::WAVES_PER_SIM
   // over the chunk costs nothing.  chunk = group gives dK/dV per kv head; smaller chunks (more
   // workgroups, for launches that would not fill the device) leave group / chunk slices to add.
   const int chunk = GROUPED ? (p.chunk > 0 ? p.chunk : p.group) : 1;
-  const TileId wg = tile_of_workgroup(p.H / chunk, p.B);  // key blocks in ascending order: most queries first
-  const int slice = wg.head, batch = wg.batch;             // output slice = chunk index
-  const int hk = slice * chunk / p.group;
+  const int pieces = PW ? 1 : imax(1, p.pieces);
+  const TileId wg = tile_of_workgroup(p.H / chunk * pieces, p.B);  // key blocks in ascending order: most queries first
+  const int slice = wg.head, batch = wg.batch;             // output slice: (chunk of heads, piece)
+  const int first_head = slice / pieces * chunk, piece = slice % pieces;
+  const int hk = first_head / p.group;
   const int M = p.M, N = p.N, pseq = N - M;
   const int n0 = wg.rank * C::BN, nw = n0 + wave * 32, my_n = nw + l32;
 
-  int head = slice * chunk;  // query head being processed
+  int head = first_head;  // query head being processed
   const T* gb = nullptr;
   const T* vb = (const T*)p.v.ptr + batch * p.v.sb + hk * p.v.sh;
   const float* lse = nullptr;
@@ -223,31 +230,37 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (KvCfg<T, D, PW, DROP>::WAVES_PER_SIM
   // registers, so a direct store would be 2 bytes per lane, 64 instructions per block.  The tiles in LDS are dead
   // by then: the wavefront rounds its block into a patch there and stores it from the patch as whole rows, 16
   // bytes per lane (8 instructions at head size 128).  Same values, same rounding.
-  auto store_keys = [&](const f32x16* acc, const View4& dst, float scale) {
-    constexpr int PLD = C::DV + 8;                       // elements per patch row: 16-byte multiples, rows 4 apart in distinct banks
-    static_assert(4 * 32 * PLD * sizeof(T) <= C::LDS_BYTES && (PLD * sizeof(T)) % 16 == 0, "four patches fit the tile stages");
-    T* patch = (T*)smem + wave * 32 * PLD;
+  auto store_keys_as = [&](auto element, const f32x16* acc, const View4& dst, float scale) {
+    using E = decltype(element);                         // T, or float for slices that are still to be added
+    constexpr int PER16 = 16 / (int)sizeof(E);           // elements of a 16-byte chunk
+    constexpr int PLD = C::DV + PER16;                   // elements per patch row: 16-byte multiples, rows 4 apart in distinct banks
+    static_assert(4 * 32 * PLD * sizeof(E) <= C::LDS_BYTES && (PLD * sizeof(E)) % 16 == 0, "four patches fit the tile stages");
+    E* patch = (E*)smem + wave * 32 * PLD;
     hw::block_sync();                                    // every wavefront has read the last operands of its last tile
 #pragma unroll
     for (int db = 0; db < C::DV / 32; ++db)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) patch[block_row(r, hh) * PLD + db * 32 + l32] = (T)(acc[db][r] * scale);
+      for (int r = 0; r < 16; ++r) patch[block_row(r, hh) * PLD + db * 32 + l32] = (E)(acc[db][r] * scale);
     hw::wave_sync();
-    T* base = (T*)dst.ptr + batch * dst.sb + slice * dst.sh;
-    constexpr int CPR = C::DV / 8, RPI = 64 / CPR;       // 16-byte chunks per row, rows per store instruction
+    E* base = (E*)dst.ptr + batch * dst.sb + slice * dst.sh;
+    constexpr int CPR = C::DV / PER16, RPI = 64 / CPR;   // 16-byte chunks per row, rows per store instruction
 #pragma unroll
     for (int i = 0; i < 32 / RPI; ++i) {
-      const int row = i * RPI + lane / CPR, d0 = (lane % CPR) * 8;
+      const int row = i * RPI + lane / CPR, d0 = (lane % CPR) * PER16;
       const int n = nw + row;
       if (n < N && d0 < D) *(u32x4*)(base + (int64_t)n * dst.st + d0) = *(const u32x4*)(patch + row * PLD + d0);
     }
     hw::block_sync();                                    // the patches are read out before a next pass writes tiles again
   };
+  auto store_keys = [&](const f32x16* acc, const View4& dst, float scale) {
+    if (!PW && p.pieces > 0) store_keys_as(float{}, acc, dst, scale);
+    else store_keys_as(T{}, acc, dst, scale);
+  };
 
   int stage = 0;
 #pragma unroll 1
   for (int gi = 0; gi < chunk; ++gi) {
-  head = slice * chunk + gi;
+  head = first_head + gi;
   gb = (const T*)p.dout.ptr + batch * p.dout.sb + head * p.dout.sh;
   lse = p.lse + ((int64_t)batch * p.H + head) * M;
   dlt = p.delta + ((int64_t)batch * p.H + head) * M;
@@ -270,6 +283,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (KvCfg<T, D, PW, DROP>::WAVES_PER_SIM
     if (PW) {
       if (far_phase) t_begin = imax(t_begin, imax(0, n0 + p.w - pseq) / C::BM);
       else t_end = imin(t_end, cdiv(imax(0, imin(M, n0 + C::BN - 1 + p.w - pseq)), C::BM));
+    } else if (pieces > 1) {
+      const int all = imax(0, t_end - t_begin);
+      t_end = t_begin + all * (piece + 1) / pieces;
+      t_begin += all * piece / pieces;
     }
     if (t_begin < t_end) {
       q_src = (const T*)(far_phase ? p.q2.ptr : p.q.ptr) + batch * (far_phase ? p.q2.sb : p.q.sb) +
@@ -728,6 +745,20 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (KvCfg<T, D, PW, DROP>::WAVES_PER_SIM
   store_keys(dv, p.dv, rp);
 }
 
+// A lane's query row of a dQ^T block (registers along D) as fp32, into slice `slice` of dst.
+template <int DV, int D>
+FA_DEVICE void store_row_slices(const f32x16* dq, const View4& dst, float scale, int batch, int slice, int my_m, int M, int hh) {
+  if (my_m >= M) return;
+  float* o = (float*)dst.ptr + batch * dst.sb + slice * dst.sh + (int64_t)my_m * dst.st;
+#pragma unroll
+  for (int db = 0; db < DV / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = db * 32 + 8 * g + 4 * hh;
+      if (d < D) *(hw::f32x4*)(o + d) = hw::f32x4{dq[db][4 * g] * scale, dq[db][4 * g + 1] * scale, dq[db][4 * g + 2] * scale, dq[db][4 * g + 3] * scale};
+    }
+}
+
 // ----------------------------------------------------------------------------------- dQ ----
 template <class T, int D, bool PW>
 struct QCfg {
@@ -742,6 +773,9 @@ struct QCfg {
   static constexpr size_t LDS_BYTES = 2 * STAGE_BYTES;
 };
 
+// Pieces (p.pieces > 0, plain attention; also of the kernel that reads dS): the key tiles of a row block are dealt to that
+// many workgroups, which leave their sums in fp32 as slices (head, piece) of p.dq; fa_sum_slices_kernel adds them.
+//
 // PW: two passes over the key tiles, as in the forward kernel -- the far keys with (q2, k2)
 // accumulating dQ2, then the near keys with (q1, k1) accumulating dQ1 in the same registers.
 // DROP: dP is masked and scaled by 1 / (1 - dropout_p) before dS = P (dP - delta) (flash.py:877-890); 1: the mask is
@@ -756,9 +790,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
 
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const TileId wg = tile_of_workgroup(p.H, p.B);
+  const int pieces = PW ? 1 : imax(1, p.pieces);
+  const TileId wg = tile_of_workgroup(p.H * pieces, p.B);
   const int mb = (p.M + C::BM - 1) / C::BM - 1 - wg.rank;  // long rows first under the causal mask
-  const int head = wg.head, batch = wg.batch;
+  const int head = wg.head / pieces, piece = wg.head % pieces, batch = wg.batch;
   const int hk = head / p.group;
   const int M = p.M, N = p.N, pseq = N - M;
   const int m0 = mb * C::BM, mw = m0 + wave * 32, my_m = mw + l32;
@@ -824,6 +859,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
 
   // dQ^T blocks: lane owns one query row, registers run along D
   auto store_rows = [&](const View4& dst) {
+    if (!PW && p.pieces > 0) {
+      store_row_slices<C::DV, D>(dq, dst, p.sm_scale, batch, wg.head, my_m, M, hh);
+      return;
+    }
     if (my_m < M) {
       T* o1 = (T*)dst.ptr + batch * dst.sb + head * dst.sh + (int64_t)my_m * dst.st;
 #pragma unroll
@@ -853,6 +892,9 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
       } else {
         t_begin = imax(0, m0 + pseq - p.w + 1) / C::BN;
       }
+    } else if (pieces > 1) {
+      t_end = n_tiles * (piece + 1) / pieces;
+      t_begin = n_tiles * piece / pieces;
     }
     if (t_begin < t_end) {
       k_src = (const T*)(far_phase ? p.k2.ptr : p.k.ptr) + batch * (far_phase ? p.k2.sb : p.k.sb) +
@@ -997,9 +1039,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_bwd_dq_from_ds_kernel(BwdParams
 
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const TileId wg = tile_of_workgroup(p.H, p.B);
+  const int pieces = PW ? 1 : imax(1, p.pieces);
+  const TileId wg = tile_of_workgroup(p.H * pieces, p.B);
   const int mb = (p.M + C::BM - 1) / C::BM - 1 - wg.rank;  // long rows first under the causal mask
-  const int head = wg.head, batch = wg.batch;
+  const int head = wg.head / pieces, piece = wg.head % pieces, batch = wg.batch;
   const int hk = head / p.group;
   const int M = p.M, N = p.N, pseq = N - M;
   const int m0 = mb * C::BM, mw = m0 + wave * 32, my_m = mw + l32;
@@ -1019,8 +1062,13 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_bwd_dq_from_ds_kernel(BwdParams
     if (far) hi = imin(hi, m0 + C::BM - 1 + pseq - p.w + 1);  // far: n <= m + pseq - w
     else lo = imax(0, m0 + pseq - p.w + 1);                    // near: n > m + pseq - w
   }
-  const int t_lo = lo / C::BN;
-  const int n_tiles = hi > lo ? cdiv(hi, C::BN) : t_lo;
+  int t_lo = lo / C::BN;
+  int n_tiles = hi > lo ? cdiv(hi, C::BN) : t_lo;
+  if (!PW && pieces > 1) {
+    const int all = n_tiles;   // from key 0 on
+    n_tiles = all * (piece + 1) / pieces;
+    t_lo = all * piece / pieces;
+  }
 
   if (C::DV != D) {
     for (int i = tid; i < (int)(C::LDS_BYTES / sizeof(T)); i += kThreads) lds[i] = (T)0.f;
@@ -1101,7 +1149,9 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_bwd_dq_from_ds_kernel(BwdParams
     stage ^= 1;
   }
 
-  if (my_m < M) {
+  if (!PW && p.pieces > 0) {
+    store_row_slices<C::DV, D>(dq, p.dq, p.sm_scale, batch, wg.head, my_m, M, hh);
+  } else if (my_m < M) {
     T* o1 = (T*)p.dq.ptr + batch * p.dq.sb + head * p.dq.sh + (int64_t)my_m * p.dq.st;
 #pragma unroll
     for (int db = 0; db < C::DV / 32; ++db)
@@ -1118,11 +1168,56 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_bwd_dq_from_ds_kernel(BwdParams
   }
 }
 
+// ------------------------------------------------------------------------- sums of slices ----
+// out[o][i] = sum over s of slices[o][s][i] for up to three tensors in one launch (grid.y), 8 elements per thread.
+// Bound by the read of the slices, four of them in flight per thread.
+template <class T>
+FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_sum_slices_kernel(SumParams p) {
+  const SumParams::Item it = p.item[hw::block_y()];
+  const int64_t first = ((int64_t)hw::block_x() * kThreads + hw::thread_id()) * 8;
+  if (first >= it.outer * it.inner) return;
+  const int64_t o = first / it.inner;
+  const float* src = it.slices + o * it.count * it.inner + (first - o * it.inner);
+  hw::f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+  constexpr int kBatch = 4;
+  for (int s0 = 0; s0 < it.count; s0 += kBatch) {
+    hw::f32x4 a[kBatch], b[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float* q = src + (int64_t)imin(s0 + u, it.count - 1) * it.inner;
+      a[u] = *(const hw::f32x4*)q;
+      b[u] = *(const hw::f32x4*)(q + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (s0 + u < it.count) { lo += a[u]; hi += b[u]; }
+  }
+  *(u32x4*)((T*)it.out + first) = u32x4{hw::pack2(T{}, lo[0], lo[1]), hw::pack2(T{}, lo[2], lo[3]),
+                                        hw::pack2(T{}, hi[0], hi[1]), hw::pack2(T{}, hi[2], hi[3])};
+}
+
+int run_sum_slices(const SumParams& p, hipStream_t stream) {
+  int64_t most = 0;
+  for (int i = 0; i < p.items; ++i) {
+    const SumParams::Item& t = p.item[i];
+    if (!t.slices || !t.out || ((((uintptr_t)t.slices) | ((uintptr_t)t.out)) & 15) || t.outer <= 0 || t.count <= 0 ||
+        t.inner <= 0 || t.inner % 8)
+      return kBadArgument;
+    most = t.outer * t.inner > most ? t.outer * t.inner : most;
+  }
+  const int64_t wgs = (most / 8 + kThreads - 1) / kThreads;
+  if (p.items <= 0 || wgs > 0x7fffffff) return kBadArgument;
+  const dim3 grid((unsigned)wgs, p.items, 1);
+  if (p.dtype == kDtypeF16) return launch(fa_sum_slices_kernel<hw::half_t>, grid, 0, stream, p);
+  if (p.dtype == kDtypeBF16) return launch(fa_sum_slices_kernel<hw::bf16_t>, grid, 0, stream, p);
+  return kUnsupported;
+}
+
 // ------------------------------------------------------------------------------ launchers ----
 template <class T, bool PW, bool DS, int DROP, bool GROUPED>
 static int launch_dkdv(const BwdParams& p, hipStream_t stream) {
   const int chunk = GROUPED ? (p.chunk > 0 ? p.chunk : p.group) : 1;
-  dim3 grid(((p.N + 127) / 128) * (p.H / chunk) * p.B, 1, 1);
+  dim3 grid(((p.N + 127) / 128) * (p.H / chunk) * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
   switch (p.D) {
     case 16: return launch(fa_bwd_dkdv_kernel<T, 16, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 16, PW, DROP>::LDS_BYTES, stream, p);
     case 32: return launch(fa_bwd_dkdv_kernel<T, 32, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 32, PW, DROP>::LDS_BYTES, stream, p);
@@ -1134,7 +1229,7 @@ static int launch_dkdv(const BwdParams& p, hipStream_t stream) {
 
 template <class T, bool PW, int DROP>
 static int launch_dq(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(((p.M + 127) / 128) * p.H * p.B, 1, 1);
+  dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
   switch (p.D) {
     case 16: return launch(fa_bwd_dq_kernel<T, 16, PW, DROP>, grid, QCfg<T, 16, PW>::LDS_BYTES, stream, p);
     case 32: return launch(fa_bwd_dq_kernel<T, 32, PW, DROP>, grid, QCfg<T, 32, PW>::LDS_BYTES, stream, p);
@@ -1148,6 +1243,7 @@ static bool bwd_args_ok(const BwdParams& p, bool piecewise) {
   if (p.B <= 0 || p.H <= 0 || p.M <= 0 || p.N <= 0 || p.group <= 0) return false;
   if (p.chunk < 0 || (p.chunk > 0 && p.group % p.chunk)) return false;
   if (!(p.dropout_p >= 0.f && p.dropout_p < 1.f) || (piecewise && p.dropout_p > 0.f)) return false;
+  if (p.pieces < 0 || p.pieces > kMaxPieces || (piecewise && p.pieces)) return false;
   return true;
 }
 
@@ -1200,7 +1296,7 @@ int run_bwd_dq(const BwdParams& a, bool piecewise, hipStream_t stream) {
 
 template <class T, bool PW>
 static int launch_dq_from_ds(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(((p.M + 127) / 128) * p.H * p.B, 1, 1);
+  dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
   switch (p.D) {
     case 16: return launch(fa_bwd_dq_from_ds_kernel<T, 16, PW>, grid, QdsCfg<T, 16>::LDS_BYTES, stream, p);
     case 32: return launch(fa_bwd_dq_from_ds_kernel<T, 32, PW>, grid, QdsCfg<T, 32>::LDS_BYTES, stream, p);
@@ -1224,7 +1320,7 @@ int run_bwd_dkdv_ds(const BwdParams& a, bool piecewise, hipStream_t stream) {
 
 // piecewise: one launch per regime (p.regime, with p.k and p.dq set to that regime's tensors)
 int run_bwd_dq_from_ds(const BwdParams& p, bool piecewise, hipStream_t stream) {
-  if (p.B <= 0 || p.H <= 0 || p.M <= 0 || p.N <= 0 || p.group <= 0 || !p.ds) return kBadArgument;
+  if (!bwd_args_ok(p, piecewise) || !p.ds) return kBadArgument;
   if (piecewise && !(p.regime == 1 || p.regime == 2)) return kBadArgument;
   if (p.dtype == kDtypeF16)
     return piecewise ? launch_dq_from_ds<hw::half_t, true>(p, stream) : launch_dq_from_ds<hw::half_t, false>(p, stream);

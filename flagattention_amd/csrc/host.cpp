@@ -105,6 +105,38 @@ int dkdv_heads_per_slice(int64_t B, int64_t H, int group, int64_t N, int cus) {
   return 1;
 }
 
+// How a backward kernel's workgroups use a compute unit: `slots` of them share it; a step (64 queries or keys) takes one
+// `alone` us, each of a full set `shared` us, and what comes before and behind the steps `around` us.  Measured on long
+// launches (shared) and on launches of less than one workgroup per unit (alone).
+struct Pace { int slots; double alone, shared, around; };
+constexpr Pace kDkdv128 = {1, 1.7, 2.1, 6.0}, kDkdv64 = {2, 1.05, 2.1, 5.0}, kDq = {2, 1.1, 1.6, 4.0}, kDqFromDs = {2, 1.15, 1.6, 4.0};
+
+// Estimated us of a launch of `tiles` result tiles of up to `steps` steps each, every tile's sum dealt to `pieces`
+// workgroups.  Under the causal mask workgroups start longest first and average half the longest.
+double launch_us(const Pace& pace, int64_t tiles, double steps, bool causal, int pieces, double slice_bytes, int cus) {
+  const double wgs = (double)tiles * pieces, per = steps / pieces, full = (double)cus * pace.slots;
+  double t;
+  if (causal) {
+    t = std::max(per * pace.alone, tiles * steps / 2 / full * pace.shared);
+  } else {
+    const double rounds = std::floor(wgs / full), rest = wgs - rounds * full;
+    t = per * (rounds * pace.shared + (rest <= 0 ? 0 : rest <= cus ? pace.alone : pace.shared));
+  }
+  t += pace.around * std::max(1.0, wgs / full);
+  return pieces == 1 ? t : t + 3.0 + 2 * wgs * slice_bytes / 5e6;   // fp32 slices written and read back at 5 TB/s, and the launch that adds them
+}
+// Workgroups that share the sum of one result tile (FA_PIECES): more than one where a launch is as long as its longest
+// workgroup, or its last round of workgroups is nearly empty, and that costs more than adding the pieces does.
+int contraction_pieces(const Pace& pace, int64_t tiles, int64_t steps, bool causal, double slice_bytes, int cus) {
+  int best = 1;
+  double least = launch_us(pace, tiles, (double)steps, causal, 1, slice_bytes, cus);
+  for (int n = 2; n <= 16 && steps >= 8 * n; ++n) {
+    const double t = launch_us(pace, tiles, (double)steps, causal, n, slice_bytes, cus);
+    if (t < 0.95 * least) { best = n; least = t; }
+  }
+  return best;
+}
+
 // flash.ds_heads_per_launch
 int64_t ds_heads_per_launch(int64_t B, int64_t H, int group, int64_t M, int64_t N, int64_t D, int64_t limit_mib, int grids) {
   if (D < 128 || M * N < 1024 * 1024 || limit_mib <= 0) return 0;
@@ -270,69 +302,91 @@ variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, c
 variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& L,
                              const Tensor& keep, const Tensor& grad, const FlashCall& c, int64_t limit_mib) {
   const int B = (int)q.size(0), H = (int)q.size(1), M = (int)q.size(2), D = (int)q.size(3);
-  const int Hk = (int)k.size(1), N = (int)k.size(2), group = H / Hk, type = dtype_code(q);
+  const int Hk = (int)k.size(1), N = (int)k.size(2), group = H / Hk, type = dtype_code(q), cus = fa_num_cus();
   const Tensor g = kernel_ready(grad);
   void* stream = stream_of(q);
-  const fa_view4 vq = view4(q), vk = view4(k), vv = view4(v), vo = view4(o), vg = view4(g);
   const float scale = (float)c.scale, p = (float)c.dropout_p;
   Tensor delta = empty(L.sizes(), at::kFloat, q);
+  const fa_view4 vo = view4(o), vg = view4(g);
   check(fa_bwd_delta(type, &vo, &vg, f32(delta), B, H, M, D, stream), "fa_bwd_delta");
-  // one slice of dK / dV per `chunk` query heads; the kernels that sum query heads are built without dropout
-  const int chunk = c.dropout_p > 0 ? 1 : dkdv_heads_per_slice(B, H, group, N, fa_num_cus());
-  const int slices = H / chunk;
-  Tensor dk = empty({B, slices, N, D}, k.scalar_type(), q), dv = empty({B, slices, N, D}, k.scalar_type(), q);
-  Tensor dq = empty({B, H, M, D}, q.scalar_type(), q);
-  const fa_view4 vdk = view4(dk), vdv = view4(dv), vdq = view4(dq);
-  int64_t heads = ds_heads_per_launch(B, H, group, M, N, D, limit_mib, 1);
+
+  // dS kept (heads > 0), for all heads in one launch pair or for `hn` heads of one batch entry at a time; or recomputed,
+  // where it is not worth keeping for this shape or there is no memory for it
+  const int64_t heads = ds_heads_per_launch(B, H, group, M, N, D, limit_mib, 1);
+  int bn = B, hn = H;   // batch entries and heads per launch
   Tensor ds;
   if (heads >= (int64_t)B * H) ds = ds_workspace(q, B, H, M, N, 1);
-  else if (heads > 0) ds = ds_workspace(q, 1, heads = std::min<int64_t>(heads, H), M, N, 1);
+  else if (heads > 0) ds = ds_workspace(q, bn = 1, hn = (int)std::min<int64_t>(heads, H), M, N, 1);
+  if (!ds.defined()) { bn = B; hn = H; }
+
+  // Slices of dK / dV: one per `chunk` query heads (the kernels that sum query heads are built without dropout) and
+  // piece of the query axis; of dQ: one per piece of the key axis.  More than one per result: fp32, added at the end.
+  const int chunk = c.dropout_p > 0 ? 1 : dkdv_heads_per_slice(bn, hn, group, N, cus);
+  // (counted over all heads, so that launches in turns add up in the same order as one launch)
+  const int kv_pieces = chunk > 1 ? 1 : contraction_pieces(D == 128 ? kDkdv128 : kDkdv64, cdiv(N, 128) * B * H, cdiv(M, 64), c.causal, 2 * 4.0 * 128 * D, cus);
+  const int q_pieces = contraction_pieces(ds.defined() ? kDqFromDs : kDq, cdiv(M, 128) * B * H, cdiv(N, 64), c.causal, 4.0 * 128 * D, cus);
+  const int kv_slices = group / chunk * kv_pieces;   // per kv head
+  Tensor dk = empty({B, Hk, N, D}, k.scalar_type(), q), dv = empty({B, Hk, N, D}, k.scalar_type(), q);
+  Tensor dq = empty({B, H, M, D}, q.scalar_type(), q), dk_s = dk, dv_s = dv, dq_s = dq;
+  int kv_type = type, q_type = type;
+  if (kv_slices > 1) {
+    dk_s = empty({B, (int64_t)Hk * kv_slices, N, D}, at::kFloat, q);
+    dv_s = empty({B, (int64_t)Hk * kv_slices, N, D}, at::kFloat, q);
+    kv_type |= FA_PIECES(kv_pieces);
+  }
+  if (q_pieces > 1) {
+    dq_s = empty({B, (int64_t)H * q_pieces, M, D}, at::kFloat, q);
+    q_type |= FA_PIECES(q_pieces);
+  }
   const uint32_t* bits = keep.defined() ? (const uint32_t*)keep.const_data_ptr() : nullptr;
-  if (!ds.defined() && bits) {
-    check(fa_bwd_dkdv_keep(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, nullptr, 0, bits, B, H, Hk, M, N, D,
-                           c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
-    check(fa_bwd_dq_keep(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdq, bits, B, H, Hk, M, N, D, c.causal, scale, p,
-                         stream), "fa_bwd_dq_keep");
-  } else if (!ds.defined()) {   // dS not worth keeping for this shape, or no memory for it: recompute it
-    check(fa_bwd_dkdv(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, B, H, Hk, M, N, D, c.causal,
-                      scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv");
-    check(fa_bwd_dq(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdq, B, H, Hk, M, N, D, c.causal, scale, p, c.seed,
-                    c.offset, stream), "fa_bwd_dq");
-  } else if (heads >= (int64_t)B * H) {
-    if (bits)
-      check(fa_bwd_dkdv_keep(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, ds.mutable_data_ptr(), ds.numel(),
-                             bits, B, H, Hk, M, N, D, c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
-    else
-      check(fa_bwd_dkdv_ds(type, &vq, &vk, &vv, &vg, f32(L), f32(delta), &vdk, &vdv, chunk, ds.mutable_data_ptr(),
-                           ds.numel(), B, H, Hk, M, N, D, c.causal, scale, p, c.seed, c.offset, stream), "fa_bwd_dkdv_ds");
-    check(fa_bwd_dq_from_ds(type, &vk, ds.const_data_ptr(), ds.numel(), &vdq, B, H, Hk, M, N, D, c.causal, scale,
-                            stream), "fa_bwd_dq_from_ds");
-  } else {
-    // bounded workspace: one batch entry and `heads` query heads (whole groups) at a time; the dropout counter of a
-    // slice starts where the slice starts in the (B, H, M, N) score tensor
-    for (int64_t b = 0; b < B; ++b)
-      for (int64_t h0 = 0; h0 < H; h0 += heads) {
-        const int n = (int)(std::min<int64_t>(H, h0 + heads) - h0), kn = n / group;
-        const fa_view4 sq = slice4(q, b, h0), sk = slice4(k, b, h0 / group), sv = slice4(v, b, h0 / group),
-                       sg = slice4(g, b, h0), sdk = slice4(dk, b, h0 / chunk), sdv = slice4(dv, b, h0 / chunk),
-                       sdq = slice4(dq, b, h0);
-        const int64_t row = (b * H + h0) * M;
-        if (bits)
-          check(fa_bwd_dkdv_keep(type, &sq, &sk, &sv, &sg, f32(L) + row, f32(delta) + row, &sdk, &sdv, ds.mutable_data_ptr(),
-                                 ds.numel(), bits + (b * H + h0) * fa_dropout_keep_words(M, N), 1, n, kn, M, N, D,
-                                 c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
-        else
-          check(fa_bwd_dkdv_ds(type, &sq, &sk, &sv, &sg, f32(L) + row, f32(delta) + row, &sdk, &sdv, chunk,
-                               ds.mutable_data_ptr(), ds.numel(), 1, n, kn, M, N, D, c.causal, scale, p, c.seed,
-                               c.offset + (uint64_t)row * (uint64_t)N, stream), "fa_bwd_dkdv_ds");
-        check(fa_bwd_dq_from_ds(type, &sk, ds.const_data_ptr(), ds.numel(), &sdq, 1, n, kn, M, N, D, c.causal, scale,
+  const int64_t head_bits = bits ? fa_dropout_keep_words(M, N) : 0;
+
+  for (int b = 0; b < B; b += bn)
+    for (int h0 = 0; h0 < H; h0 += hn) {
+      const int n = std::min(H, h0 + hn) - h0, kn = n / group, k0 = h0 / group;   // whole groups of query heads
+      const fa_view4 vq = slice4(q, b, h0), vk = slice4(k, b, k0), vv = slice4(v, b, k0), vg = slice4(g, b, h0),
+                     vdk = slice4(dk_s, b, (int64_t)k0 * kv_slices), vdv = slice4(dv_s, b, (int64_t)k0 * kv_slices),
+                     vdq = slice4(dq_s, b, (int64_t)h0 * q_pieces);
+      const int64_t row = ((int64_t)b * H + h0) * M;
+      const float *l = f32(L) + row, *d = f32(delta) + row;
+      const uint32_t* w = bits ? bits + ((int64_t)b * H + h0) * head_bits : nullptr;
+      // the dropout counter of a launch starts where its heads start in the (B, H, M, N) score tensor
+      const uint64_t offset = c.offset + (uint64_t)row * (uint64_t)N;
+      if (bits)
+        check(fa_bwd_dkdv_keep(kv_type, &vq, &vk, &vv, &vg, l, d, &vdk, &vdv, ds.defined() ? ds.mutable_data_ptr() : nullptr,
+                               ds.defined() ? ds.numel() : 0, w, bn, n, kn, M, N, D, c.causal, scale, p, stream), "fa_bwd_dkdv_keep");
+      else if (ds.defined())
+        check(fa_bwd_dkdv_ds(kv_type, &vq, &vk, &vv, &vg, l, d, &vdk, &vdv, chunk, ds.mutable_data_ptr(), ds.numel(), bn, n,
+                             kn, M, N, D, c.causal, scale, p, c.seed, offset, stream), "fa_bwd_dkdv_ds");
+      else
+        check(fa_bwd_dkdv(kv_type, &vq, &vk, &vv, &vg, l, d, &vdk, &vdv, chunk, bn, n, kn, M, N, D, c.causal, scale, p,
+                          c.seed, offset, stream), "fa_bwd_dkdv");
+      if (ds.defined())
+        check(fa_bwd_dq_from_ds(q_type, &vk, ds.const_data_ptr(), ds.numel(), &vdq, bn, n, kn, M, N, D, c.causal, scale,
                                 stream), "fa_bwd_dq_from_ds");
-      }
-  }
-  if (slices > Hk) {   // the kernel summed `chunk` heads of every group; add the chunks
-    dk = dk.view({B, Hk, slices / Hk, N, D}).sum(2);
-    dv = dv.view({B, Hk, slices / Hk, N, D}).sum(2);
-  }
+      else if (bits)
+        check(fa_bwd_dq_keep(q_type, &vq, &vk, &vv, &vg, l, d, &vdq, w, bn, n, kn, M, N, D, c.causal, scale, p, stream),
+              "fa_bwd_dq_keep");
+      else
+        check(fa_bwd_dq(q_type, &vq, &vk, &vv, &vg, l, d, &vdq, bn, n, kn, M, N, D, c.causal, scale, p, c.seed, offset,
+                        stream), "fa_bwd_dq");
+    }
+
+  const float* slices[3];
+  void* out[3];
+  int64_t outer[3], inner[3];
+  int32_t count[3];
+  int sums = 0;
+  auto add_up = [&](const Tensor& s, const Tensor& r, int n) {
+    slices[sums] = f32(s);
+    out[sums] = r.mutable_data_ptr();
+    outer[sums] = r.size(0) * r.size(1);
+    inner[sums] = r.size(2) * r.size(3);
+    count[sums++] = n;
+  };
+  if (kv_slices > 1) { add_up(dk_s, dk, kv_slices); add_up(dv_s, dv, kv_slices); }
+  if (q_pieces > 1) add_up(dq_s, dq, q_pieces);
+  if (sums) check(fa_sum_slices(type, slices, out, outer, count, inner, sums, stream), "fa_sum_slices");
   return {dq, dk, dv};
 }
 

@@ -52,6 +52,7 @@ struct BwdParams {
   float dropout_p;
   uint32_t threshold;     // dropout_threshold(dropout_p), filled in by the launchers
   uint64_t seed, offset;
+  int pieces;             // > 0: results as fp32 slices, the contraction of each dealt to that many workgroups
   const uint32_t* keep;   // the forward's mask, or null: drawn again from (seed, offset)
 };
 
@@ -144,6 +145,14 @@ struct ProbeParams {
 int run_probe_mfma(const ProbeParams& p, hipStream_t stream);
 
 inline int64_t dropout_keep_words(int M, int N) { return 64 * (int64_t)((M + 31) / 32) * ((N + 63) / 64); }   // per (batch, head)
+constexpr int kMaxPieces = 64;
+
+struct SumParams {   // out (outer, inner) of the call's dtype = sum of slices (outer, count, inner), fp32, contiguous
+  struct Item { const float* slices; void* out; int64_t outer, inner; int count; } item[3];
+  int items;
+  int dtype;
+};
+int run_sum_slices(const SumParams& p, hipStream_t stream);
 int64_t bwd_ds_workspace_bytes(int B, int H, int M, int N);
 int run_bwd_dkdv_ds(const BwdParams& p, bool piecewise, hipStream_t stream);
 int run_bwd_dq_from_ds(const BwdParams& p, bool piecewise, hipStream_t stream);

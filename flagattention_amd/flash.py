@@ -212,14 +212,6 @@ class FlashAttention(torch.autograd.Function):
             backward_settings(B, H, M, N, D, causal)
             delta = torch.empty_like(L)
             _abi.fa_bwd_delta(lib, o, do, delta)
-            # dK/dV come out summed over each kv head's group of query heads (flash.py:205-206,250-251
-            # of the reference produce one slice per query head and reduce afterwards)
-            # the kernels that sum query heads are built without dropout
-            chunk = 1 if dropout[0] > 0 else dkdv_heads_per_slice(B, H, group, N, _num_cus())
-            slices = H // chunk
-            dk = torch.empty((B, slices, N, D), dtype=k.dtype, device=q.device)
-            dv = torch.empty((B, slices, N, D), dtype=v.dtype, device=q.device)
-            dq = torch.empty((B, H, M, D), dtype=q.dtype, device=q.device)
             heads = ds_heads_per_launch(lib, B, H, group, M, N, D)
             ds = None
             if heads >= B * H:
@@ -227,11 +219,23 @@ class FlashAttention(torch.autograd.Function):
             elif heads > 0:
                 heads = min(heads, H)
                 ds = _ds_workspace(lib, q.device, 1, heads, M, N)
+            # dK/dV come out summed over each kv head's group of query heads (flash.py:205-206,250-251
+            # of the reference produce one slice per query head and reduce afterwards), or over chunks of
+            # it, then as fp32 slices that are added below
+            # the kernels that sum query heads are built without dropout
+            in_turns = ds is not None and heads < B * H     # launches of one batch entry and `heads` heads
+            chunk = 1 if dropout[0] > 0 else dkdv_heads_per_slice(1 if in_turns else B, heads if in_turns else H,
+                                                                  group, N, _num_cus())
+            slices = H // chunk
+            pieces = 1 if slices > Hk else 0
+            dk = torch.empty((B, slices, N, D), dtype=torch.float32 if pieces else k.dtype, device=q.device)
+            dv = torch.empty((B, slices, N, D), dtype=torch.float32 if pieces else v.dtype, device=q.device)
+            dq = torch.empty((B, H, M, D), dtype=q.dtype, device=q.device)
             if ds is None:   # dS not worth keeping for this shape, or no memory for it: recompute it
-                _abi.fa_bwd_dkdv(lib, q, k, v, do, L, delta, dk, dv, causal, sm_scale, dropout)
+                _abi.fa_bwd_dkdv(lib, q, k, v, do, L, delta, dk, dv, causal, sm_scale, dropout, pieces)
                 _abi.fa_bwd_dq(lib, q, k, v, do, L, delta, dq, causal, sm_scale, dropout)
             elif heads >= B * H:
-                _abi.fa_bwd_dkdv_ds(lib, q, k, v, do, L, delta, dk, dv, ds, causal, sm_scale, dropout)
+                _abi.fa_bwd_dkdv_ds(lib, q, k, v, do, L, delta, dk, dv, ds, causal, sm_scale, dropout, pieces)
                 _abi.fa_bwd_dq_from_ds(lib, k, ds, dq, causal, sm_scale)
             else:
                 # bounded workspace: one batch entry and `heads` query heads at a time; the dropout
@@ -244,11 +248,12 @@ class FlashAttention(torch.autograd.Function):
                         bs = slice(b, b + 1)
                         drop = (dropout[0], dropout[1], dropout[2] + (b * H + h0) * M * N)
                         _abi.fa_bwd_dkdv_ds(lib, q[bs, hs], k[bs, ks], v[bs, ks], do[bs, hs], L[bs, hs],
-                                            delta[bs, hs], dk[bs, ss], dv[bs, ss], ds, causal, sm_scale, drop)
+                                            delta[bs, hs], dk[bs, ss], dv[bs, ss], ds, causal, sm_scale, drop, pieces)
                         _abi.fa_bwd_dq_from_ds(lib, k[bs, ks], ds, dq[bs, hs], causal, sm_scale)
-            if slices > Hk:   # the kernel summed `chunk` heads of every group; add the chunks
-                dk = dk.reshape(B, Hk, slices // Hk, N, D).sum(2)
-                dv = dv.reshape(B, Hk, slices // Hk, N, D).sum(2)
+            if pieces:   # the kernel summed `chunk` heads of every group; add the chunks
+                parts = dk, dv
+                dk, dv = (torch.empty((B, Hk, N, D), dtype=k.dtype, device=q.device) for _ in parts)
+                _abi.fa_sum_slices(lib, parts, (dk, dv))
         return dq, dk, dv, None, None, None, None, None, None
 
 
@@ -258,7 +263,7 @@ def dkdv_heads_per_slice(B, H, group, N, num_cus):
     the launch still has at least two workgroups per compute unit (with fewer, the unequal lengths of
     the workgroups under the causal mask cannot be balanced: 3.0 instead of 1.9 ms at 32 query / 4 kv
     heads, T = 8192), otherwise the largest divisor of the group that gets there; the remaining
-    slices are added with one torch sum."""
+    slices are fp32 and added by a kernel of their own.  ``B`` and ``H`` are those of one launch."""
     blocks = -(-N // 128)
     for chunk in range(group, 0, -1):
         if group % chunk == 0 and blocks * B * (H // chunk) >= 2 * num_cus:

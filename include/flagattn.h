@@ -135,6 +135,16 @@ int fa_bwd_dq_keep(int dtype, const fa_view4* q, const fa_view4* k, const fa_vie
                    const float* lse, const float* delta, const fa_view4* dq, const uint32_t* keep, int B, int H, int Hk,
                    int M, int N, int D, int causal, float sm_scale, float dropout_p, void* stream);
 
+/* Gradients in pieces.  `dtype | FA_PIECES(n)`, n = 1 .. 64, in fa_bwd_dkdv, fa_bwd_dkdv_ds, fa_bwd_dkdv_keep,
+ * fa_bwd_dq, fa_bwd_dq_keep and fa_bwd_dq_from_ds: the sum that makes up a tile of the result is dealt to n workgroups
+ * (a launch of too few, too long ones otherwise), and dk / dv / dq are fp32 with n slices in place of each one --
+ * (B, H / heads_per_slice * n, N, D) and (B, H * n, M, D), slice n * i + piece -- that are still to be added.
+ * fa_sum_slices adds them: out[t] (outer, inner) of `dtype` = sum over slices[t] (outer, count, inner), all contiguous,
+ * 16-byte aligned, inner a multiple of 8, for up to three tensors in one launch (the arrays are read on the host). */
+#define FA_PIECES(n) ((n) << 8)
+int fa_sum_slices(int dtype, const float* const* slices, void* const* out, const int64_t* outer, const int32_t* count,
+                  const int64_t* inner, int tensors, void* stream);
+
 /* ------------------------------------------------------------------------- total attention --
  * Replaces `_total_attention_kernel` (src/flag_attn/total.py:50-142; launches flash.py:128-140 and
  * total.py:35-46): total[b,h,n] = sum_m softmax(scores)[m,n], recomputed from q, k and lse. */

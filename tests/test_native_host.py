@@ -48,7 +48,7 @@ def same(a, b):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,Hk,M,N,D,causal,layout", [
-    (1, 32, 8, 1, 1024, 128, True, "BHTD"),       # split decode
+    (1, 32, 8, 1, 1024, 128, True, "BHTD"),       # split decode; gradients of a group added
     (1, 8, 8, 1, 1030, 64, False, "BTHD"),        # decode in one piece: no merge
     (1, 32, 8, 300, 5000, 128, True, "BTHD"),     # pieces of the key axis through the 256-row kernel
     (2, 4, 4, 513, 511, 64, False, "BHTD"),       # dense; recomputing backward
@@ -62,8 +62,10 @@ def test_native_flash_equals_the_python_path(B, H, Hk, M, N, D, causal, layout):
     for a, b in zip(native[:3], python[:3]):
         assert same(a, b)
     assert native[3:] == (None, None)
+    # (the native backward may deal a sum to several workgroups: another order of fp32 additions, one rounding to bf16)
     for a, b in zip(torch.autograd.grad(native[0], (q, k, v), do), torch.autograd.grad(python[0], (q, k, v), do)):
-        assert same(a, b)
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert (a.float() - b.float()).abs().max() <= 2 ** -7 * b.float().abs().max()
     with torch.no_grad():
         assert torch.equal(flag_attn.flash_attention(q, k, v, causal), native[0])
 
