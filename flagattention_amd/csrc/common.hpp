@@ -13,6 +13,7 @@
 #include <utility>
 
 #include "hw.hpp"
+#include "params.hpp"
 
 namespace fa {
 
@@ -141,9 +142,28 @@ FA_DEVICE typename hw::Elem<T>::v8 operand_transposed(const T* lds_tile, int t0,
 // tail (balanced finish under the causal mask); and because consecutive ids go to consecutive XCDs,
 // a given (batch, head) -- whose K/V or Q/dO every one of its tiles re-reads -- stays on one XCD's
 // L2 whenever batch * heads is a multiple of the XCD count.
+//
+// `deal`: where a compute unit holds several workgroups, the first of a launch are all resident from the start, in
+// rounds of one per unit, and unit i gets workgroup i of every round.  Ranked by length throughout, the unit with the
+// longest tile would also hold the longest of the second round: 32768 rows of 2 heads under the causal mask (512
+// workgroups of 128 rows on 256 units) give one unit 512 + 256 steps and the last one 258 + 2.  Odd rounds therefore run
+// from short to long, and where the second round is not full, the longest of the first go to units of their own.
+// Workgroups move by multiples of 8, so a head keeps its XCD.  dQ from dS at that size 605 -> 551 us per launch; the
+// step of B=4 H=16 T=1024 D=64 with dropout (512 workgroups per launch) 127 -> 120 us.
 struct TileId { int rank, head, batch; };
-FA_DEVICE TileId tile_of_workgroup(int H, int B) {
-  const int lin = hw::block_x(), bh = lin % (H * B);
+FA_DEVICE int dealt(int lin, int grid, Deal deal) {
+  if (deal.resident < 2 || grid <= deal.unit) return lin;
+  const int unit = deal.unit, round = lin / unit;
+  if (round == 0 && grid < 2 * unit) {
+    const int shared = (grid - unit) & ~7;   // units with a second workgroup
+    return lin < shared ? lin + unit - shared : lin - shared;
+  }
+  if (round >= deal.resident || !(round & 1)) return lin;
+  const int begin = round * unit, end = (begin + unit < grid ? begin + unit : grid) & ~7;
+  return lin < end ? begin + end - 8 - (lin & ~7) + (lin & 7) : lin;
+}
+FA_DEVICE TileId tile_of_workgroup(int H, int B, Deal deal = Deal{0, 0}) {
+  const int lin = dealt(hw::block_x(), hw::grid_x(), deal), bh = lin % (H * B);
   TileId t;
   t.rank = lin / (H * B);
   t.head = bh % H;
@@ -288,6 +308,34 @@ int launch(void (*kern)(P), dim3 grid, size_t lds_bytes, hipStream_t stream, con
   }
   hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, stream, p);
   return (int)hipGetLastError();
+}
+
+// Workgroups of a kernel that a compute unit of the current device holds; asked once per kernel and device.
+template <class P>
+int resident_workgroups(void (*kern)(P), size_t lds_bytes) {
+  static std::mutex lock;
+  static std::unordered_map<const void*, int> known[kMaxDevices];
+  int dev = -1, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 1;
+  std::lock_guard<std::mutex> g(lock);
+  auto it = known[dev].find((const void*)kern);
+  if (it != known[dev].end()) return it->second;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)kern, kThreads, lds_bytes) != hipSuccess) return 1;
+  return known[dev][(const void*)kern] = n;
+}
+
+// A launch whose tiles differ in length under the causal mask: the kernel deals them by tile_of_workgroup.
+template <class P>
+int launch_dealt(void (*kern)(P), dim3 grid, size_t lds_bytes, hipStream_t stream, P p) {
+  const int unit = num_cus_of_current_device();
+  if (p.causal && unit > 0 && unit % 8 == 0 && (int64_t)grid.x > unit) {
+    if (lds_bytes > 48 * 1024) {
+      const int rc = allow_lds(kern, lds_bytes);
+      if (rc) return rc;
+    }
+    p.deal = Deal{unit, resident_workgroups(kern, lds_bytes)};
+  }
+  return launch(kern, grid, lds_bytes, stream, p);
 }
 
 // error codes of the C entry points (positive values are hipError_t)

@@ -128,7 +128,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (KvCfg<T, D, PW, DROP>::WAVES_PER_SIM
   // workgroups, for launches that would not fill the device) leave group / chunk slices to add.
   const int chunk = GROUPED ? (p.chunk > 0 ? p.chunk : p.group) : 1;
   const int pieces = PW ? 1 : imax(1, p.pieces);
-  const TileId wg = tile_of_workgroup(p.H / chunk * pieces, p.B);  // key blocks in ascending order: most queries first
+  const TileId wg = tile_of_workgroup(p.H / chunk * pieces, p.B, p.deal);  // key blocks in ascending order: most queries first
   const int slice = wg.head, batch = wg.batch;             // output slice: (chunk of heads, piece)
   const int first_head = slice / pieces * chunk, piece = slice % pieces;
   const int hk = first_head / p.group;
@@ -791,7 +791,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (QCfg<T, D, PW>::WAVES_PER_SIMD)) fa_
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int pieces = PW ? 1 : imax(1, p.pieces);
-  const TileId wg = tile_of_workgroup(p.H * pieces, p.B);
+  const TileId wg = tile_of_workgroup(p.H * pieces, p.B, p.deal);
   const int mb = (p.M + C::BM - 1) / C::BM - 1 - wg.rank;  // long rows first under the causal mask
   const int head = wg.head / pieces, piece = wg.head % pieces, batch = wg.batch;
   const int hk = head / p.group;
@@ -1040,7 +1040,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_bwd_dq_from_ds_kernel(BwdParams
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int pieces = PW ? 1 : imax(1, p.pieces);
-  const TileId wg = tile_of_workgroup(p.H * pieces, p.B);
+  const TileId wg = tile_of_workgroup(p.H * pieces, p.B, p.deal);
   const int mb = (p.M + C::BM - 1) / C::BM - 1 - wg.rank;  // long rows first under the causal mask
   const int head = wg.head / pieces, piece = wg.head % pieces, batch = wg.batch;
   const int hk = head / p.group;
@@ -1219,10 +1219,10 @@ static int launch_dkdv(const BwdParams& p, hipStream_t stream) {
   const int chunk = GROUPED ? (p.chunk > 0 ? p.chunk : p.group) : 1;
   dim3 grid(((p.N + 127) / 128) * (p.H / chunk) * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
   switch (p.D) {
-    case 16: return launch(fa_bwd_dkdv_kernel<T, 16, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 16, PW, DROP>::LDS_BYTES, stream, p);
-    case 32: return launch(fa_bwd_dkdv_kernel<T, 32, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 32, PW, DROP>::LDS_BYTES, stream, p);
-    case 64: return launch(fa_bwd_dkdv_kernel<T, 64, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 64, PW, DROP>::LDS_BYTES, stream, p);
-    case 128: return launch(fa_bwd_dkdv_kernel<T, 128, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 128, PW, DROP>::LDS_BYTES, stream, p);
+    case 16: return launch_dealt(fa_bwd_dkdv_kernel<T, 16, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 16, PW, DROP>::LDS_BYTES, stream, p);
+    case 32: return launch_dealt(fa_bwd_dkdv_kernel<T, 32, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 32, PW, DROP>::LDS_BYTES, stream, p);
+    case 64: return launch_dealt(fa_bwd_dkdv_kernel<T, 64, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 64, PW, DROP>::LDS_BYTES, stream, p);
+    case 128: return launch_dealt(fa_bwd_dkdv_kernel<T, 128, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 128, PW, DROP>::LDS_BYTES, stream, p);
   }
   return kUnsupported;
 }
@@ -1231,10 +1231,10 @@ template <class T, bool PW, int DROP>
 static int launch_dq(const BwdParams& p, hipStream_t stream) {
   dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
   switch (p.D) {
-    case 16: return launch(fa_bwd_dq_kernel<T, 16, PW, DROP>, grid, QCfg<T, 16, PW>::LDS_BYTES, stream, p);
-    case 32: return launch(fa_bwd_dq_kernel<T, 32, PW, DROP>, grid, QCfg<T, 32, PW>::LDS_BYTES, stream, p);
-    case 64: return launch(fa_bwd_dq_kernel<T, 64, PW, DROP>, grid, QCfg<T, 64, PW>::LDS_BYTES, stream, p);
-    case 128: return launch(fa_bwd_dq_kernel<T, 128, PW, DROP>, grid, QCfg<T, 128, PW>::LDS_BYTES, stream, p);
+    case 16: return launch_dealt(fa_bwd_dq_kernel<T, 16, PW, DROP>, grid, QCfg<T, 16, PW>::LDS_BYTES, stream, p);
+    case 32: return launch_dealt(fa_bwd_dq_kernel<T, 32, PW, DROP>, grid, QCfg<T, 32, PW>::LDS_BYTES, stream, p);
+    case 64: return launch_dealt(fa_bwd_dq_kernel<T, 64, PW, DROP>, grid, QCfg<T, 64, PW>::LDS_BYTES, stream, p);
+    case 128: return launch_dealt(fa_bwd_dq_kernel<T, 128, PW, DROP>, grid, QCfg<T, 128, PW>::LDS_BYTES, stream, p);
   }
   return kUnsupported;
 }
@@ -1298,10 +1298,10 @@ template <class T, bool PW>
 static int launch_dq_from_ds(const BwdParams& p, hipStream_t stream) {
   dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
   switch (p.D) {
-    case 16: return launch(fa_bwd_dq_from_ds_kernel<T, 16, PW>, grid, QdsCfg<T, 16>::LDS_BYTES, stream, p);
-    case 32: return launch(fa_bwd_dq_from_ds_kernel<T, 32, PW>, grid, QdsCfg<T, 32>::LDS_BYTES, stream, p);
-    case 64: return launch(fa_bwd_dq_from_ds_kernel<T, 64, PW>, grid, QdsCfg<T, 64>::LDS_BYTES, stream, p);
-    case 128: return launch(fa_bwd_dq_from_ds_kernel<T, 128, PW>, grid, QdsCfg<T, 128>::LDS_BYTES, stream, p);
+    case 16: return launch_dealt(fa_bwd_dq_from_ds_kernel<T, 16, PW>, grid, QdsCfg<T, 16>::LDS_BYTES, stream, p);
+    case 32: return launch_dealt(fa_bwd_dq_from_ds_kernel<T, 32, PW>, grid, QdsCfg<T, 32>::LDS_BYTES, stream, p);
+    case 64: return launch_dealt(fa_bwd_dq_from_ds_kernel<T, 64, PW>, grid, QdsCfg<T, 64>::LDS_BYTES, stream, p);
+    case 128: return launch_dealt(fa_bwd_dq_from_ds_kernel<T, 128, PW>, grid, QdsCfg<T, 128>::LDS_BYTES, stream, p);
   }
   return kUnsupported;
 }

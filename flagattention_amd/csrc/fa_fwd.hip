@@ -44,7 +44,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
 
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const TileId wg = tile_of_workgroup(p.H, p.B);
+  const TileId wg = tile_of_workgroup(p.H, p.B, p.deal);
   const int mb = (p.M + C::BM - 1) / C::BM - 1 - wg.rank;  // long rows first under the causal mask
   const int head = wg.head, batch = wg.batch;
   const int hk = head / p.group;
@@ -292,10 +292,10 @@ template <class T, bool PW, bool DROP>
 static int launch_fwd(const FwdParams& p, hipStream_t stream) {
   dim3 grid(((p.M + 127) / 128) * p.H * p.B, 1, 1);
   switch (p.D) {
-    case 16: return launch(fa_fwd_kernel<T, 16, PW, DROP>, grid, FwdCfg<T, 16, PW>::LDS_BYTES, stream, p);
-    case 32: return launch(fa_fwd_kernel<T, 32, PW, DROP>, grid, FwdCfg<T, 32, PW>::LDS_BYTES, stream, p);
-    case 64: return launch(fa_fwd_kernel<T, 64, PW, DROP>, grid, FwdCfg<T, 64, PW>::LDS_BYTES, stream, p);
-    case 128: return launch(fa_fwd_kernel<T, 128, PW, DROP>, grid, FwdCfg<T, 128, PW>::LDS_BYTES, stream, p);
+    case 16: return launch_dealt(fa_fwd_kernel<T, 16, PW, DROP>, grid, FwdCfg<T, 16, PW>::LDS_BYTES, stream, p);
+    case 32: return launch_dealt(fa_fwd_kernel<T, 32, PW, DROP>, grid, FwdCfg<T, 32, PW>::LDS_BYTES, stream, p);
+    case 64: return launch_dealt(fa_fwd_kernel<T, 64, PW, DROP>, grid, FwdCfg<T, 64, PW>::LDS_BYTES, stream, p);
+    case 128: return launch_dealt(fa_fwd_kernel<T, 128, PW, DROP>, grid, FwdCfg<T, 128, PW>::LDS_BYTES, stream, p);
   }
   return kUnsupported;
 }

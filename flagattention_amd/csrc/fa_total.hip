@@ -28,7 +28,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_total_kernel(TotalParams p) {
 
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const TileId wg = tile_of_workgroup(p.H, p.B);  // key blocks in ascending order: most queries first
+  const TileId wg = tile_of_workgroup(p.H, p.B, p.deal);  // key blocks in ascending order: most queries first
   const int head = wg.head, batch = wg.batch;
   const int hk = head / p.group;
   const int M = p.M, N = p.N, pseq = N - M;
@@ -112,10 +112,10 @@ template <class T>
 static int launch_total(const TotalParams& p, hipStream_t stream) {
   dim3 grid(((p.N + 127) / 128) * p.H * p.B, 1, 1);
   switch (p.D) {
-    case 16: return launch(fa_total_kernel<T, 16>, grid, TotCfg<T, 16>::LDS_BYTES, stream, p);
-    case 32: return launch(fa_total_kernel<T, 32>, grid, TotCfg<T, 32>::LDS_BYTES, stream, p);
-    case 64: return launch(fa_total_kernel<T, 64>, grid, TotCfg<T, 64>::LDS_BYTES, stream, p);
-    case 128: return launch(fa_total_kernel<T, 128>, grid, TotCfg<T, 128>::LDS_BYTES, stream, p);
+    case 16: return launch_dealt(fa_total_kernel<T, 16>, grid, TotCfg<T, 16>::LDS_BYTES, stream, p);
+    case 32: return launch_dealt(fa_total_kernel<T, 32>, grid, TotCfg<T, 32>::LDS_BYTES, stream, p);
+    case 64: return launch_dealt(fa_total_kernel<T, 64>, grid, TotCfg<T, 64>::LDS_BYTES, stream, p);
+    case 128: return launch_dealt(fa_total_kernel<T, 128>, grid, TotCfg<T, 128>::LDS_BYTES, stream, p);
   }
   return kUnsupported;
 }

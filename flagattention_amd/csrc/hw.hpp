@@ -38,6 +38,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 FA_DEVICE int thread_id() { return (int)threadIdx.x; }
 FA_DEVICE int block_x() { return (int)blockIdx.x; }
+FA_DEVICE int grid_x() { return (int)gridDim.x; }
 FA_DEVICE int block_y() { return (int)blockIdx.y; }
 FA_DEVICE int block_z() { return (int)blockIdx.z; }
 FA_DEVICE int grid_z() { return (int)gridDim.z; }

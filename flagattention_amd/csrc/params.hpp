@@ -11,6 +11,10 @@ struct View4 {
   int64_t sb, sh, st;
 };
 
+// The first workgroups of a launch under the causal mask, which are all resident at once, and the compute units they
+// share: `resident` rounds of `unit` workgroups (0: no such order).  See tile_of_workgroup.
+struct Deal { int unit, resident; };
+
 struct FwdParams {
   View4 q, k, v, q2, k2;  // q2/k2 only for the piecewise variant
   View4 o;                // written
@@ -32,6 +36,7 @@ struct FwdParams {
   int num_splits, split_size;
   void* part_o;
   float* part_lse;
+  Deal deal;              // filled in at the launch
 };
 
 struct BwdParams {
@@ -54,6 +59,7 @@ struct BwdParams {
   uint64_t seed, offset;
   int pieces;             // > 0: results as fp32 slices, the contraction of each dealt to that many workgroups
   const uint32_t* keep;   // the forward's mask, or null: drawn again from (seed, offset)
+  Deal deal;              // filled in at the launch
 };
 
 struct TotalParams {
@@ -65,6 +71,7 @@ struct TotalParams {
   int causal;
   float sm_scale;
   int dtype;
+  Deal deal;         // filled in at the launch
 };
 
 }  // namespace fa

@@ -36,6 +36,7 @@ enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount };
 inline hipError_t hipGetDevice(int* dev) { *dev = 0; return hipSuccess; }
 inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
 inline hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+template <class K> hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, K, int, size_t) { *n = 2; return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipGetSymbolAddress(void** p, const void* symbol) { *p = const_cast<void*>(symbol); return hipSuccess; }
 #define HIP_SYMBOL(x) (&(x))
@@ -241,6 +242,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 inline int thread_id() { return hwsim::cur; }
 inline int block_x() { return hwsim::bx; }
+inline int grid_x() { return hwsim::gx; }
 inline int block_y() { return hwsim::by; }
 inline int block_z() { return hwsim::bz; }
 inline void store_streaming(void* p, u32x4 v) { *(u32x4*)p = v; }
