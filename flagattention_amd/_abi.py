@@ -88,6 +88,16 @@ def fa_fwd(lib, q, k, v, o, lse, causal, sm_scale, dropout=NO_DROPOUT, block_m=0
                      _u64(dropout[2]), int(block_m), stream_of(q)), "fa_fwd")
 
 
+def fa_fwd_pieces(lib, q, k, v, o, lse, causal, sm_scale, pieces):
+    """The 128-row kernel with the keys of every row block dealt to ``pieces`` workgroups, and the merge."""
+    B, H, M, D = q.shape
+    Hk, N = k.shape[1], k.shape[2]
+    workspace = torch.empty(B * H * pieces * M * (D + 1), dtype=torch.float32, device=q.device)
+    check(lib.fa_fwd_pieces(dtype_code(q), view4(q), view4(k), view4(v), view4(o), ptr(lse), ptr(workspace),
+                            workspace.numel() * 4, B, H, Hk, M, N, D, int(causal), float(sm_scale), int(pieces),
+                            stream_of(q)), "fa_fwd_pieces")
+
+
 def fa_fwd_keep(lib, q, k, v, o, lse, keep, causal, sm_scale, dropout):
     """Forward with dropout that leaves its mask in ``keep`` (int32, B * H * fa_dropout_keep_words(M, N))."""
     B, H, M, D = q.shape

@@ -24,6 +24,7 @@ SIGNATURES = {
     "fa_version": [],
     "fa_num_cus": [],
     "fa_fwd": [_i, _v, _v, _v, _v, _p, _i, _i, _i, _i, _i, _i, _i, _f, _f, _u64, _u64, _i, _p],
+    "fa_fwd_pieces": [_i, _v, _v, _v, _v, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _i, _f, _i, _p],
     "fa_dropout_keep_words": [_i, _i],
     "fa_fwd_keep": [_i, _v, _v, _v, _v, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _f, _u64, _u64, _p],
     "fa_bwd_dkdv_keep": [_i, _v, _v, _v, _v, _p, _p, _v, _v, _p, _i64, _p, _i, _i, _i, _i, _i, _i, _i, _f, _f, _p],

@@ -71,6 +71,32 @@ int fa_fwd(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, c
   return fa::run_fwd(p, false, (hipStream_t)stream);
 }
 
+int fa_fwd_pieces(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* o, float* lse,
+                  void* workspace, int64_t workspace_bytes, int B, int H, int Hk, int M, int N, int D, int causal,
+                  float sm_scale, int pieces, void* stream) {
+  if (!view_ok(q) || !view_ok(k) || !view_ok(v) || !view_ok(o) || !lse || !workspace) return FA_ERR_BAD_ARGUMENT;
+  if (((uintptr_t)workspace) & 15) return FA_ERR_BAD_ARGUMENT;
+  if (!head_dim_ok(D)) return FA_ERR_UNSUPPORTED;
+  if (Hk <= 0 || H % Hk || B <= 0 || M <= 0 || N <= 0 || pieces < 1 || pieces > 64) return FA_ERR_BAD_ARGUMENT;
+  if ((int64_t)((M + 127) / 128) * B * H * pieces > 0x7fffffff) return FA_ERR_BAD_ARGUMENT;
+  if (workspace_bytes < (int64_t)B * H * pieces * M * (D + 1) * (int64_t)sizeof(float)) return FA_ERR_BAD_ARGUMENT;
+  fa::FwdParams p = {};
+  p.q = to_view(q); p.k = to_view(k); p.v = to_view(v); p.o = to_view(o);
+  p.lse = lse;
+  p.B = B; p.H = H; p.M = M; p.N = N; p.D = D;
+  p.group = H / Hk;
+  p.causal = causal; p.sm_scale = sm_scale; p.dtype = dtype;
+  p.block_m = 128; p.num_splits = pieces;
+  p.part_o = workspace;   // (B, H, pieces, M, D), then the log-normalizers
+  p.part_lse = (float*)workspace + (int64_t)B * H * pieces * M * D;
+  const int rc = fa::run_fwd(p, false, (hipStream_t)stream);
+  if (rc) return rc;
+  fa::CombineParams c = {};
+  c.part_o = p.part_o; c.part_lse = p.part_lse; c.o = p.o; c.lse = lse;
+  c.B = B; c.H = H; c.M = M; c.D = D; c.num_splits = pieces; c.dtype = dtype; c.f32 = true;
+  return fa::run_combine(c, (hipStream_t)stream);
+}
+
 int fa_dropout_keep_words(int M, int N) {
   if (M <= 0 || N <= 0) return FA_ERR_BAD_ARGUMENT;
   const int64_t words = fa::dropout_keep_words(M, N);

@@ -32,6 +32,11 @@ struct FwdCfg {
   static constexpr size_t LDS_BYTES = 2 * STAGE * sizeof(T);
 };
 
+// Pieces (p.num_splits > 0, plain attention): the key tiles of a row block are dealt to that many workgroups, each of
+// which leaves its normalised output in fp32 and its log-normalizer for fa_combine_kernel.  For launches of fewer
+// workgroups than the device holds, which are as long as one walk over the keys (about 1 us per 64 of them):
+// 32 heads, 100 rows, 8200 keys, D=128 162 us whole, 36 in 8 pieces; the rule is flash.forward_pieces.
+//
 // DROP: dropout as in the reference (flash.py:450-457, 479-482): the row sum is taken before the mask,
 // dropped probabilities do not enter the second product, the output is scaled by 1 / (1 - dropout_p).
 template <class T, int D, bool PW, bool DROP = false>
@@ -44,9 +49,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
 
   const int tid = hw::thread_id(), lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const TileId wg = tile_of_workgroup(p.H, p.B, p.deal);
+  const int pieces = PW || DROP ? 1 : imax(1, p.num_splits);
+  const TileId wg = tile_of_workgroup(p.H * pieces, p.B, p.deal);
   const int mb = (p.M + C::BM - 1) / C::BM - 1 - wg.rank;  // long rows first under the causal mask
-  const int head = wg.head, batch = wg.batch;
+  const int head = wg.head / pieces, piece = wg.head % pieces, batch = wg.batch;
   const int hk = head / p.group;
   const int M = p.M, N = p.N, pseq = N - M;
   const int m0 = mb * C::BM, mw = m0 + wave * 32, my_m = mw + l32;
@@ -236,6 +242,9 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
       } else {          // keys n > m0 + pseq - w are near some row
         t_begin = imax(0, m0 + pseq - p.w + 1) / C::BN;
       }
+    } else if (pieces > 1) {
+      t_begin = n_tiles * piece / pieces;
+      t_end = n_tiles * (piece + 1) / pieces;
     }
     if (t_begin >= t_end) continue;
     k_src = far_phase ? k2b : kb;
@@ -269,7 +278,22 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
   const float l_tot = l_i + hw::xor32(l_i);
   const bool empty = !(l_tot > 0.f);
   const float inv = empty ? 0.f : (DROP ? 1.f / ((1.f - p.dropout_p) * l_tot) : 1.f / l_tot);
-  if (my_m < M) {
+  if (!(PW || DROP) && p.num_splits > 0) {
+    if (my_m >= M) return;
+    const int64_t slot = (((int64_t)batch * p.H + head) * pieces + piece) * M + my_m;
+    float* ob = (float*)p.part_o + slot * D;
+#pragma unroll
+    for (int db = 0; db < C::DV / 32; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = db * 32 + 8 * g + 4 * hh;
+        if (d < D) {
+          const float w[4] = {oacc[db][4 * g + 0] * inv, oacc[db][4 * g + 1] * inv, oacc[db][4 * g + 2] * inv, oacc[db][4 * g + 3] * inv};
+          *(u32x4*)(ob + d) = __builtin_bit_cast(u32x4, w);
+        }
+      }
+    if (hh == 0) p.part_lse[slot] = empty ? neg_inf() : m_i * p.sm_scale + hw::log_nat(l_tot);
+  } else if (my_m < M) {
     T* ob = (T*)p.o.ptr + batch * p.o.sb + head * p.o.sh + (int64_t)my_m * p.o.st;
 #pragma unroll
     for (int db = 0; db < C::DV / 32; ++db)
@@ -290,7 +314,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
 
 template <class T, bool PW, bool DROP>
 static int launch_fwd(const FwdParams& p, hipStream_t stream) {
-  dim3 grid(((p.M + 127) / 128) * p.H * p.B, 1, 1);
+  dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.num_splits > 0 ? p.num_splits : 1), 1, 1);
   switch (p.D) {
     case 16: return launch_dealt(fa_fwd_kernel<T, 16, PW, DROP>, grid, FwdCfg<T, 16, PW>::LDS_BYTES, stream, p);
     case 32: return launch_dealt(fa_fwd_kernel<T, 32, PW, DROP>, grid, FwdCfg<T, 32, PW>::LDS_BYTES, stream, p);
@@ -316,6 +340,7 @@ static bool prefer_wide(const FwdParams& p) {
 int run_fwd(const FwdParams& p, bool piecewise, hipStream_t stream) {
   if (p.B <= 0 || p.H <= 0 || p.M <= 0 || p.N < 0 || p.group <= 0) return kBadArgument;
   if (!(p.dropout_p >= 0.f && p.dropout_p < 1.f) || (piecewise && p.dropout_p > 0.f)) return kBadArgument;
+  if (p.num_splits > 0 && (piecewise || p.dropout_p > 0.f || p.block_m != 128 || !p.part_o || !p.part_lse)) return kBadArgument;
   if (p.block_m != 0 && p.block_m != 128 && p.block_m != 256) return kUnsupported;
   if (p.block_m == 256 && (piecewise || !fwd_wide_supported(p))) return kUnsupported;
   if (!piecewise && (p.block_m == 256 || (p.block_m == 0 && fwd_wide_supported(p) && prefer_wide(p)))) return run_fwd_wide(p, stream);

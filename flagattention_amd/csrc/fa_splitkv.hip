@@ -91,8 +91,9 @@ struct CombineCfg {
   static constexpr int GROUPS = SPREAD ? 64 / LANES : 1;
   static constexpr int ROWS = kThreads / (LANES * GROUPS);
 };
-template <class T, int D, int BATCH, bool SPREAD>
+template <class T, int D, int BATCH, bool SPREAD, class P>   // P: type of the partial outputs, fp16 or float
 FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_combine_kernel(CombineParams p) {
+  constexpr int WORDS = (int)sizeof(P) / 2;                  // 16-byte loads for the 8 elements
   using C = CombineCfg<T, D, BATCH, SPREAD>;
   const int tid = hw::thread_id(), group = tid / C::LANES % C::GROUPS;
   const int64_t total_rows = (int64_t)p.B * p.H * p.M;
@@ -114,12 +115,14 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_combine_kernel(CombineParams p) {
   };
   for (int s0 = group * BATCH; s0 < S; s0 += C::GROUPS * BATCH) {
     float l[BATCH];
-    u32x4 raw[BATCH];
+    u32x4 raw[BATCH][WORDS];
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
       const int s = imin(s0 + u, S - 1);
       l[u] = ls[(int64_t)s * p.M];
-      raw[u] = *(const u32x4*)((const hw::half_t*)p.part_o + ((bh * S + s) * p.M + m) * D + col);
+      const u32x4* part = (const u32x4*)((const P*)p.part_o + ((bh * S + s) * p.M + m) * D + col);
+#pragma unroll
+      for (int w = 0; w < WORDS; ++w) raw[u][w] = part[w];
     }
     float t = top;
 #pragma unroll
@@ -130,9 +133,14 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_combine_kernel(CombineParams p) {
       if (s0 + u >= S || l[u] == neg_inf()) continue;  // past the end, or a split without a visible key
       const float wgt = hw::exp2_fast((l[u] - top) * kLog2e);
       z += wgt;
-      auto v = hw::as_v8<hw::half_t>(raw[u]);
+      if constexpr (WORDS == 2) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] += wgt * (float)v[e];
+        for (int e = 0; e < 8; ++e) acc[e] += wgt * __builtin_bit_cast(float, (uint32_t)raw[u][e / 4][e % 4]);
+      } else {
+        auto v = hw::as_v8<hw::half_t>(raw[u][0]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += wgt * (float)v[e];
+      }
     }
   }
   if constexpr (C::GROUPS > 1) {
@@ -184,16 +192,20 @@ int run_splitkv(const SplitParams& p, hipStream_t stream) {
   return kUnsupported;
 }
 
-template <class T, int D>
-static int launch_combine_d(const CombineParams& p, hipStream_t stream) {
+template <class T, int D, class P>
+static int launch_combine_as(const CombineParams& p, hipStream_t stream) {
   const int64_t total = (int64_t)p.B * p.H * p.M;
   auto go = [&](auto kern, auto cfg) {
     using C = decltype(cfg);
     return launch(kern, dim3((unsigned)((total + C::ROWS - 1) / C::ROWS)), 0, stream, p);
   };
-  if (p.num_splits <= 4) return go(fa_combine_kernel<T, D, 4, false>, CombineCfg<T, D, 4, false>{});
-  if (p.num_splits <= 8) return go(fa_combine_kernel<T, D, 8, false>, CombineCfg<T, D, 8, false>{});
-  return go(fa_combine_kernel<T, D, 8, true>, CombineCfg<T, D, 8, true>{});
+  if (p.num_splits <= 4) return go(fa_combine_kernel<T, D, 4, false, P>, CombineCfg<T, D, 4, false>{});
+  if (p.num_splits <= 8) return go(fa_combine_kernel<T, D, 8, false, P>, CombineCfg<T, D, 8, false>{});
+  return go(fa_combine_kernel<T, D, 8, true, P>, CombineCfg<T, D, 8, true>{});
+}
+template <class T, int D>
+static int launch_combine_d(const CombineParams& p, hipStream_t stream) {
+  return p.f32 ? launch_combine_as<T, D, float>(p, stream) : launch_combine_as<T, D, hw::half_t>(p, stream);
 }
 
 template <class T>

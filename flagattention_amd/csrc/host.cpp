@@ -97,6 +97,24 @@ int wide_key_splits(int64_t B, int64_t H, int64_t M, int64_t N, int64_t D, int c
   return pieces < 2 || 4 * pieces * wgs < 3 * (int64_t)cus ? 1 : (int)pieces;
 }
 
+// flash.forward_pieces (the reasons and figures stand there)
+int forward_pieces(int64_t B, int64_t H, int64_t Hk, int64_t M, int64_t N, int64_t D, bool split, int cus) {
+  if (M <= kDecodeMaxRows || (D == 128 && cdiv(M, 256) * H * B >= cus)) return 0;
+  const int64_t wgs = cdiv(M, 128) * H * B, steps = cdiv(N, 64);
+  const double alone = D == 128 ? 1.3 : D == 64 ? 0.93 : 0.75, shared = D == 128 ? 0.8 : D == 64 ? 0.45 : 0.36;
+  const double decode = D == 128 ? 2.4e-3 : D == 64 ? 0.85e-3 : 0.3e-3;
+  auto us = [&](int64_t pieces) {
+    const int64_t per_unit = cdiv(wgs * pieces, cus);
+    const double t = (double)cdiv(steps, pieces) * (alone + shared * (double)(per_unit - 1)) + 2.0 * (double)per_unit;
+    return pieces == 1 ? t : t + 6.0 + (double)(B * H * M * pieces * D * 8) / 5e6;
+  };
+  int best = 0;
+  double least = split ? 5.0 + (double)(B * Hk * cdiv(H / Hk * M, 16) * cdiv(N, 32)) * decode : us(1);
+  for (int pieces = 2; pieces <= 32 && steps >= 3 * pieces && wgs * pieces <= 4 * (int64_t)cus; ++pieces)
+    if (us(pieces) < 0.93 * least) { best = pieces; least = us(pieces); }
+  return best;
+}
+
 // flash.dkdv_heads_per_slice
 int dkdv_heads_per_slice(int64_t B, int64_t H, int group, int64_t N, int cus) {
   const int64_t blocks = cdiv(N, 128);
@@ -201,15 +219,20 @@ bool fits_int(std::initializer_list<int64_t> xs) {
   return true;
 }
 
+// memory that a slower way does without: an undefined tensor when the allocator has none left
+Tensor scratch(at::IntArrayRef shape, at::ScalarType type, const Tensor& like) {
+  try {
+    return empty(shape, type, like);
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
+}
+
 // dS of `heads` heads, or an undefined tensor when the allocator has no memory left (the caller then recomputes)
 Tensor ds_workspace(const Tensor& like, int64_t B, int64_t H, int64_t M, int64_t N, int grids) {
   const int mib = fa_bwd_ds_workspace_mib((int)B, (int)H, (int)M, (int)N);
   if (mib <= 0) check(mib ? mib : FA_ERR_BAD_ARGUMENT, "fa_bwd_ds_workspace_mib");
-  try {
-    return empty({(int64_t)grids * ((int64_t)mib << 20)}, at::kByte, like);
-  } catch (const c10::OutOfMemoryError&) {
-    return Tensor();
-  }
+  return scratch({(int64_t)grids * ((int64_t)mib << 20)}, at::kByte, like);
 }
 
 // The settings a backward reads when it runs: calls the (replaceable) tile hook, returns the dS workspace limit.
@@ -231,21 +254,25 @@ struct FlashCall {
   uint64_t seed, offset;
 };
 
-// pieces > 0: the split kernel over that many pieces of the key axis and the merge; 0: the dense kernel
-struct FlashPlan { int pieces; };
+// pieces > 0: the split kernel over that many pieces of the key axis and the merge; tiles > 0: the 128-row kernel, the
+// keys of every row block dealt to that many workgroups, and the merge; otherwise the dense kernel
+struct FlashPlan { int pieces, tiles; };
 
 // false: the combination is an error (dropout on a split shape)
 bool plan_flash(FlashPlan& plan, int64_t B, int64_t H, int64_t Hk, int64_t M, int64_t N, int64_t D, bool dropout,
                 double scale, int64_t row_bytes, int cus) {
   const int splits = num_splits_heuristic(B, H, M, N, cus, 128);
-  plan.pieces = 0;
+  plan.pieces = plan.tiles = 0;
   if (splits > 1 && dropout) return false;
+  if (splits > 1) plan.tiles = forward_pieces(B, H, Hk, M, N, D, true, cus);
+  if (plan.tiles > 0) return true;
   if (splits > 1 || (M <= kDecodeMaxRows && N >= 1024 && !dropout)) {
     plan.pieces = choose_num_splits(B, H, Hk, M, N, cus);
   } else if (!dropout && scale > 0 && row_bytes < (1 << 24)) {
     const int pieces = wide_key_splits(B, H, M, N, D, cus);
     if (pieces > 1) plan.pieces = pieces;
   }
+  if (!dropout && plan.pieces == 0) plan.tiles = forward_pieces(B, H, Hk, M, N, D, false, cus);
   return true;
 }
 
@@ -280,7 +307,11 @@ variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, c
     o = empty_result(q);
     L = empty({B, H, M}, at::kFloat, q);
     const fa_view4 vo = view4(o);
-    if (keep && c.dropout_p > 0 && keeps_mask(N, D)) {
+    const Tensor ws = plan.tiles > 0 ? scratch({(int64_t)B * H * plan.tiles * M * (D + 1)}, at::kFloat, q) : Tensor();
+    if (ws.defined()) {
+      check(fa_fwd_pieces(type, &vq, &vk, &vv, &vo, f32(L), ws.mutable_data_ptr(), ws.numel() * 4, B, H, Hk, M, N, D, c.causal,
+                          (float)c.scale, plan.tiles, stream), "fa_fwd_pieces");
+    } else if (keep && c.dropout_p > 0 && keeps_mask(N, D)) {
       *keep = empty({(int64_t)B * H * fa_dropout_keep_words(M, N)}, at::kInt, q);
       check(fa_fwd_keep(type, &vq, &vk, &vv, &vo, f32(L), (uint32_t*)keep->mutable_data_ptr(), B, H, Hk, M, N, D, c.causal,
                         (float)c.scale, (float)c.dropout_p, c.seed, c.offset, stream), "fa_fwd_keep");
@@ -682,6 +713,14 @@ PyObject* decisions(PyObject*, PyObject* args) {
   END_HANDLE_TH_ERRORS
 }
 
+// forward_pieces(B, H, Hk, M, N, D, split, num_cus), for the same test
+PyObject* pieces_of_forward(PyObject*, PyObject* args) {
+  long long B, H, Hk, M, N, D, cus;
+  int split;
+  if (!PyArg_ParseTuple(args, "LLLLLLpL", &B, &H, &Hk, &M, &N, &D, &split, &cus)) return nullptr;
+  return PyLong_FromLong(forward_pieces(B, H, Hk, M, N, D, split, (int)cus));
+}
+
 // bind(abi.check, flash settings, piecewise settings)
 PyObject* bind(PyObject*, PyObject* args) {
   if (!PyArg_ParseTuple(args, "OOO", &g_check, &g_flash_settings, &g_piecewise_settings)) return nullptr;
@@ -694,6 +733,7 @@ PyMethodDef kMethods[] = {
     {"piecewise", (PyCFunction)(void*)piecewise, METH_FASTCALL, nullptr},
     {"paged", (PyCFunction)(void*)paged, METH_FASTCALL, nullptr},
     {"decisions", decisions, METH_VARARGS, nullptr},
+    {"forward_pieces", pieces_of_forward, METH_VARARGS, nullptr},
     {"bind", bind, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -30,9 +30,10 @@ struct FwdParams {
   uint64_t seed, offset;
   uint32_t* keep;         // optional: the drawn mask for the backward (KeepMask in common.hpp)
   int block_m;            // query rows per workgroup: 128, 256, or 0 = the library's choice
-  // 256-row kernel over pieces of the key axis (0 = the whole axis, results to o / lse): piece s covers keys
-  // s * split_size .. + split_size - 1 and leaves its normalised output as fp16 in part_o (B, H, num_splits, M, D)
-  // and its log-normalizer in part_lse (B, H, num_splits, M), the layout fa_combine_kernel merges
+  // pieces of the key axis (0 = the whole axis, results to o / lse), each of which leaves its normalised output in part_o
+  // (B, H, num_splits, M, D) and its log-normalizer in part_lse (B, H, num_splits, M), the layout fa_combine_kernel
+  // merges.  256-row kernel: piece s covers keys s * split_size .. + split_size - 1, part_o is fp16; 128-row kernel: the
+  // 64-key tiles of every row block are dealt out evenly, part_o is fp32
   int num_splits, split_size;
   void* part_o;
   float* part_lse;
@@ -114,6 +115,7 @@ struct CombineParams {
   float* lse;  // (B, H, M)
   int B, H, M, D, num_splits;
   int dtype;
+  bool f32;     // part_o is fp32, otherwise fp16
 };
 
 struct PagedParams {

@@ -59,6 +59,37 @@ def wide_key_splits(B, H, M, N, D, num_cus):
     return pieces
 
 
+def forward_pieces(B, H, Hk, M, N, D, split, num_cus):
+    """Workgroups that share the keys of each 128-row block (``fa_fwd_pieces``), 0 = leave the launch as it is.
+
+    A launch of fewer workgroups than the device holds is as long as one walk over the keys: about 1 us per 64 of
+    them, whatever the rest of the device does.  ``us`` estimates a launch: the steps of a piece times the pace at which
+    a compute unit with that many workgroups advances, 2 us around them, and for more than one piece the merge (6 us) with
+    its fp32 partial results at 5 TB/s.  ``split``: the alternative is not the whole-axis launch but the decode kernel, which
+    serves 16 rows of a kv head per workgroup and reads the keys once for each 16.  Paces as measured (us per 64 keys,
+    one workgroup per unit: 1.3, 0.93, 0.75 at head size 128, 64, 32); a piece keeps at least 3 steps and a launch at
+    most 4 workgroups per unit, which bounds the partial results to 64 MiB.  us per call, before and after: 1 x 32/8
+    heads, 100 rows, 8200 keys, D=128 162 -> 36; 300 rows, 64/8 heads, 20000 keys, D=64 284 -> 156; 128 rows, 8 heads,
+    16000 keys, D=128 (decode kernel) 82 -> 28; 513 rows, 511 keys, 8 heads, D=64 stay whole (13)."""
+    if M <= DECODE_MAX_ROWS or (D == 128 and -(-M // 256) * H * B >= num_cus):   # the latter: 256-row workgroups fill the device
+        return 0
+    wgs, steps = -(-M // 128) * H * B, -(-N // 64)
+    alone, shared, decode = {128: (1.3, 0.8, 2.4e-3), 64: (0.93, 0.45, 0.85e-3)}.get(D, (0.75, 0.36, 0.3e-3))
+
+    def us(pieces):
+        per_unit = -(-wgs * pieces // num_cus)
+        t = -(-steps // pieces) * (alone + shared * (per_unit - 1)) + 2.0 * per_unit
+        return t if pieces == 1 else t + 6.0 + B * H * M * pieces * D * 8 / 5e6
+
+    best, least = 0, 5.0 + B * Hk * -(-(H // Hk * M) // 16) * -(-N // 32) * decode if split else us(1)
+    for pieces in range(2, 33):
+        if steps < 3 * pieces or wgs * pieces > 4 * num_cus:
+            break
+        if us(pieces) < 0.93 * least:
+            best, least = pieces, us(pieces)
+    return best
+
+
 _NUM_CUS = {}
 
 
@@ -146,7 +177,10 @@ class FlashAttention(torch.autograd.Function):
             splits = num_splits_heuristic(B, H, M, N, split_block_m, split_block_n, num_cus, 128)
             if splits > 1:
                 assert not is_dropout, "Cannot apply dropout with splitkv."   # as flash.py:89
-            if splits > 1 or (M <= DECODE_MAX_ROWS and N >= 1024 and not is_dropout):
+            tiles = 0   # workgroups per row block and key axis of the 128-row kernel, where that is the faster launch
+            if splits > 1 and not _hooks_replaced():
+                tiles = forward_pieces(B, H, Hk, M, N, D, True, num_cus)
+            if tiles == 0 and (splits > 1 or (M <= DECODE_MAX_ROWS and N >= 1024 and not is_dropout)):
                 o, L = split_kv_forward(lib, q, k, v, causal, sm_scale, splits)
             else:
                 # looked up by name at call time, so that an assignment to flash.get_fwd_config takes effect
@@ -159,6 +193,8 @@ class FlashAttention(torch.autograd.Function):
                     block_m = 0
                     if not is_dropout and sm_scale > 0 and max(k.stride(2), v.stride(2)) * k.element_size() < 1 << 24:
                         pieces = wide_key_splits(B, H, M, N, D, num_cus)
+                    if splits == 1 and pieces == 1 and not is_dropout:
+                        tiles = forward_pieces(B, H, Hk, M, N, D, False, num_cus)
                 elif block_m == 256 and not wide_forward_applies(D, dropout_p):
                     _config.warn_once(("fwd-wide", D, is_dropout),
                                       "flash_attention forward: the 256-row kernel is built for head size 128 "
@@ -174,14 +210,17 @@ class FlashAttention(torch.autograd.Function):
                                       "flash_attention forward: the 256-row kernel addresses key/value rows less "
                                       "than 16 MiB apart; launching the 128-row kernel")
                     block_m = 128
-                if pieces > 1:   # too few 256-row workgroups for the device: one per piece of the key axis, then the merge
+                if tiles == 0 and pieces > 1:   # too few 256-row workgroups for the device: one per piece of the key axis, then the merge
                     o, L = split_kv_forward(lib, q, k, v, causal, sm_scale, pieces, exact=True)
                 else:
                     o = torch.empty_like(q)
                     if not _abi.is_kernel_ready(o):
                         o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
                     L = torch.empty((B, H, M), device=q.device, dtype=torch.float32)
-                    _abi.fa_fwd(lib, q, k, v, o, L, causal, sm_scale, dropout, block_m)
+                    if tiles > 0:
+                        _abi.fa_fwd_pieces(lib, q, k, v, o, L, causal, sm_scale, tiles)
+                    else:
+                        _abi.fa_fwd(lib, q, k, v, o, L, causal, sm_scale, dropout, block_m)
             tot_attn = None
             if return_total_attention:
                 tot_attn = _total_attention(lib, q, k, L, causal, sm_scale)

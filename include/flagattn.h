@@ -70,7 +70,14 @@ int fa_fwd(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, c
            float* lse, int B, int H, int Hk, int M, int N, int D, int causal, float sm_scale,
            float dropout_p, uint64_t seed, uint64_t offset, int block_m, void* stream);
 
-/* The same with dropout whose mask is kept for the backward (no counterpart in the reference, whose backward kernels
+/* fa_fwd without dropout by the 128-row kernel, the keys of every row block dealt to `pieces` workgroups (1 .. 64): for
+ * launches of too few, too long ones otherwise.  workspace: B * H * pieces * M * (D + 1) floats, 16-byte aligned; its
+ * contents on entry do not matter.  The partial results in it are fp32 and merged by a second launch. */
+int fa_fwd_pieces(int dtype, const fa_view4* q, const fa_view4* k, const fa_view4* v, const fa_view4* o, float* lse,
+                  void* workspace, int64_t workspace_bytes, int B, int H, int Hk, int M, int N, int D, int causal,
+                  float sm_scale, int pieces, void* stream);
+
+/* fa_fwd with dropout whose mask is kept for the backward (no counterpart in the reference, whose backward kernels
  * draw it again, flash.py:697-721, 877-890: drawing is two to three times the work of the rest of a kernel).
  * dropout_p > 0.  keep: B * H * fa_dropout_keep_words(M, N) 32-bit words (one bit per score), 4-byte aligned, in a private
  * order; its contents on entry do not matter. */
