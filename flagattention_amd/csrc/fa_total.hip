@@ -20,8 +20,13 @@ struct TotCfg {
   static constexpr size_t LDS_BYTES = 2 * STAGE_BYTES;
 };
 
+// Bound by the vector ALU: an element takes a multiply-add, an exponential and an addition (16 clocks of issue) against 16
+// of the matrix pipe at head size 128.  The bound of two wavefronts per SIMD (four fit) makes the compiler accumulate in
+// VGPRs: in AGPRs every element is moved once more.  B=1 32/8 heads M=1000 N=8200 causal: 97 -> 83 us at D=128 (0.65 -> 0.76
+// PFLOP/s), 68 -> 50 at D=64, with the mask's branch below; two key blocks per wavefront (operands of LDS shared)
+// leave two wavefronts per SIMD of four and took 104.
 template <class T, int D>
-FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_total_kernel(TotalParams p) {
+FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_total_kernel(TotalParams p) {
   using C = TotCfg<T, D>;
   using V8 = typename hw::Elem<T>::v8;
   FA_LDS_DECL(smem);
@@ -93,12 +98,16 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_total_kernel(TotalParams p) {
         s = hw::mfma32(operand_rowmajor<T, C::LD>(sQ, sb * 32, 16 * kk, lane), kreg[kk], s);
       const bool need_mask = p.causal && (mr0 + pseq < nw + 31);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int ml = sb * 32 + block_row(r, hh);
-        float pv = hw::exp2_fast(fmaf(s[r], c2, -sL[ml]));
-        if (need_mask) pv = (m0 + ml + pseq >= my_n) ? pv : 0.f;
-        colsum += pv;
+      for (int r = 0; r < 16; ++r) s[r] = hw::exp2_fast(fmaf(s[r], c2, -sL[sb * 32 + block_row(r, hh)]));
+      // A branch of its own: left to itself the compiler makes the mask part of every block, at 5 instructions per element
+      // to the 4 that an element needs.  (A select behind the exponential: of a row without keys L is -inf.)
+      if (need_mask) {
+        hw::keep_branch();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = (mr0 + block_row(r, hh) + pseq >= my_n) ? s[r] : 0.f;
       }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) colsum += s[r];
     }
     if (more) commit((it + 1) & 1);
     hw::block_sync();
