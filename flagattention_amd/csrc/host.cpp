@@ -15,6 +15,8 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -212,6 +214,21 @@ bool is_operand(const Tensor& t, const Tensor& first) {
   return t.is_cuda() && t.dim() == 4 && t.layout() == at::kStrided && t.device() == first.device() &&
          t.scalar_type() == first.scalar_type();
 }
+// The operators' kernels are launched past the dispatcher.  Where something listens there -- a tracer, a functorch
+// transform, a dispatch mode, a tensor subclass, forward-mode tangents -- the Python form takes the call, and does with it
+// what torch does with a Python autograd function: records it or refuses it.
+bool plain_call(std::initializer_list<const Tensor*> ts) {
+  using c10::impl::tls_is_dispatch_key_included;
+  if (tls_is_dispatch_key_included(c10::DispatchKey::Tracer) ||
+      tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || c10::impl::TorchDispatchModeTLS::any_modes_set())
+    return false;
+  for (const Tensor* t : ts)
+    if (t->unsafeGetTensorImpl()->key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                                                          c10::DispatchKey::FuncTorchGradWrapper})) ||
+        t->_fw_grad(0).defined())
+      return false;
+  return true;
+}
 bool type_ok(const Tensor& t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16; }
 bool fits_int(std::initializer_list<int64_t> xs) {
   for (int64_t x : xs)
@@ -311,8 +328,8 @@ variable_list flash_forward(const Tensor& q, const Tensor& k, const Tensor& v, c
     if (ws.defined()) {
       check(fa_fwd_pieces(type, &vq, &vk, &vv, &vo, f32(L), ws.mutable_data_ptr(), ws.numel() * 4, B, H, Hk, M, N, D, c.causal,
                           (float)c.scale, plan.tiles, stream), "fa_fwd_pieces");
-    } else if (keep && c.dropout_p > 0 && keeps_mask(N, D)) {
-      *keep = empty({(int64_t)B * H * fa_dropout_keep_words(M, N)}, at::kInt, q);
+    } else if (keep && c.dropout_p > 0 && keeps_mask(N, D) &&
+               (*keep = scratch({(int64_t)B * H * fa_dropout_keep_words(M, N)}, at::kInt, q)).defined()) {
       check(fa_fwd_keep(type, &vq, &vk, &vv, &vo, f32(L), (uint32_t*)keep->mutable_data_ptr(), B, H, Hk, M, N, D, c.causal,
                         (float)c.scale, (float)c.dropout_p, c.seed, c.offset, stream), "fa_fwd_keep");
     } else {
@@ -352,22 +369,31 @@ variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, 
 
   // Slices of dK / dV: one per `chunk` query heads (the kernels that sum query heads are built without dropout) and
   // piece of the query axis; of dQ: one per piece of the key axis.  More than one per result: fp32, added at the end.
-  const int chunk = c.dropout_p > 0 ? 1 : dkdv_heads_per_slice(bn, hn, group, N, cus);
+  int chunk = c.dropout_p > 0 ? 1 : dkdv_heads_per_slice(bn, hn, group, N, cus);
   // (counted over all heads, so that launches in turns add up in the same order as one launch)
-  const int kv_pieces = chunk > 1 ? 1 : contraction_pieces(D == 128 ? kDkdv128 : kDkdv64, cdiv(N, 128) * B * H, cdiv(M, 64), c.causal, 2 * 4.0 * 128 * D, cus);
-  const int q_pieces = contraction_pieces(ds.defined() ? kDqFromDs : kDq, cdiv(M, 128) * B * H, cdiv(N, 64), c.causal, 4.0 * 128 * D, cus);
-  const int kv_slices = group / chunk * kv_pieces;   // per kv head
+  int kv_pieces = chunk > 1 ? 1 : contraction_pieces(D == 128 ? kDkdv128 : kDkdv64, cdiv(N, 128) * B * H, cdiv(M, 64), c.causal, 2 * 4.0 * 128 * D, cus);
+  int q_pieces = contraction_pieces(ds.defined() ? kDqFromDs : kDq, cdiv(M, 128) * B * H, cdiv(N, 64), c.causal, 4.0 * 128 * D, cus);
+  int kv_slices = group / chunk * kv_pieces;   // per kv head
   Tensor dk = empty({B, Hk, N, D}, k.scalar_type(), q), dv = empty({B, Hk, N, D}, k.scalar_type(), q);
   Tensor dq = empty({B, H, M, D}, q.scalar_type(), q), dk_s = dk, dv_s = dv, dq_s = dq;
   int kv_type = type, q_type = type;
   if (kv_slices > 1) {
-    dk_s = empty({B, (int64_t)Hk * kv_slices, N, D}, at::kFloat, q);
-    dv_s = empty({B, (int64_t)Hk * kv_slices, N, D}, at::kFloat, q);
-    kv_type |= FA_PIECES(kv_pieces);
+    dk_s = scratch({B, (int64_t)Hk * kv_slices, N, D}, at::kFloat, q);
+    if (dk_s.defined()) dv_s = scratch({B, (int64_t)Hk * kv_slices, N, D}, at::kFloat, q);
+    if (!dk_s.defined() || !dv_s.defined()) {   // no memory: whole sums, by as few slices as there are kernels for
+      TORCH_CHECK_WITH(OutOfMemoryError, chunk == group || c.dropout_p == 0, "flash_attention backward: no memory for the slices of dK and dV");
+      chunk = group;
+      kv_pieces = kv_slices = 1;
+      dk_s = dk;
+      dv_s = dv;
+    } else {
+      kv_type |= FA_PIECES(kv_pieces);
+    }
   }
   if (q_pieces > 1) {
-    dq_s = empty({B, (int64_t)H * q_pieces, M, D}, at::kFloat, q);
-    q_type |= FA_PIECES(q_pieces);
+    dq_s = scratch({B, (int64_t)H * q_pieces, M, D}, at::kFloat, q);
+    if (dq_s.defined()) q_type |= FA_PIECES(q_pieces);
+    else { q_pieces = 1; dq_s = dq; }
   }
   const uint32_t* bits = keep.defined() ? (const uint32_t*)keep.const_data_ptr() : nullptr;
   const int64_t head_bits = bits ? fa_dropout_keep_words(M, N) : 0;
@@ -479,7 +505,7 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int causal = PyObject_IsTrue(a[3]), want_lse = PyObject_IsTrue(a[6]), want_total = PyObject_IsTrue(a[7]),
             want_seed = PyObject_IsTrue(a[8]);
   if (causal < 0 || want_lse < 0 || want_total < 0 || want_seed < 0) throw python_error();
-  if (!is_operand(q, q) || !is_operand(k, q) || !is_operand(v, q) || !type_ok(q)) return not_taken();
+  if (!plain_call({&q, &k, &v}) || !is_operand(q, q) || !is_operand(k, q) || !is_operand(v, q) || !type_ok(q)) return not_taken();
   const int64_t B = q.size(0), H = q.size(1), M = q.size(2), D = q.size(3), Hk = k.size(1), N = k.size(2);
   if (!fits_int({B, H, M, N, Hk}) || k.size(0) != B || v.sizes() != k.sizes() || k.size(3) != D || H % Hk ||
       !(D == 16 || D == 32 || D == 64 || D == 128))
@@ -609,6 +635,7 @@ PyObject* piecewise(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!THPVariable_Check(a[i])) return not_taken();
   const Tensor &q1 = THPVariable_Unpack(a[0]), &k1 = THPVariable_Unpack(a[1]), &q2 = THPVariable_Unpack(a[2]),
                &k2 = THPVariable_Unpack(a[3]), &v = THPVariable_Unpack(a[4]);
+  if (!plain_call({&q1, &k1, &q2, &k2, &v})) return not_taken();
   for (const Tensor* t : {&q1, &k1, &q2, &k2, &v})
     if (!is_operand(*t, q1)) return not_taken();
   const int64_t D = q1.size(3);

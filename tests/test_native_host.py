@@ -128,3 +128,34 @@ def test_native_piecewise_equals_the_python_path(T, D, w):
     assert same(a, b)
     for x, y in zip(torch.autograd.grad(a, ins, do), torch.autograd.grad(b, ins, do)):
         assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["flash", "piecewise"])
+def test_transforms_and_tracers_see_a_python_function(op):
+    """Forward-mode tangents, functorch transforms and the tracer meet the same function that they would without the native
+    path: what torch refuses is refused, and a trace holds the call and not its results."""
+    from torch.autograd import forward_ad
+    if op == "flash":
+        native, python = (lambda *t: flag_attn.flash_attention(*t[:3], True)), \
+            (lambda *t: flash.FlashAttention.apply(*t[:3], True, None, 0.0, False, False, False))
+    else:
+        native, python = (lambda *t: flag_attn.piecewise_attention(*t, 40, True)), \
+            (lambda *t: piecewise.PiecewiseAttention.apply(*t, 40, True, None))
+    ins, others = ([randn(1, 2, 96, 64) for _ in range(5)] for _ in range(2))
+
+    def tangents(f):
+        with forward_ad.dual_level():
+            return f(*[forward_ad.make_dual(t, torch.ones_like(t)) for t in ins])
+
+    def outcome(f):
+        try:
+            return f()
+        except Exception as e:   # noqa: BLE001 - compared below
+            return type(e)
+    for form in (tangents, lambda f: torch.func.grad(lambda q: f(q, *ins[1:]).sum())(ins[0]),
+                 lambda f: torch.vmap(lambda q: f(q, *ins[1:]))(torch.stack([ins[0]] * 2)),
+                 lambda f: torch.jit.trace(f, tuple(ins), check_trace=False)(*others)):
+        a, b = outcome(lambda: form(native)), outcome(lambda: form(python))
+        assert isinstance(a, torch.Tensor) == isinstance(b, torch.Tensor), (a, b)
+        assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a is b, (a, b)
