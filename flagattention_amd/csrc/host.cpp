@@ -165,6 +165,12 @@ int64_t ds_heads_per_launch(int64_t B, int64_t H, int group, int64_t M, int64_t 
   return fit >= B * H ? B * H : fit / group * group;
 }
 
+// flash.even_heads
+int64_t even_heads(int64_t fit, int64_t H, int group) {
+  const int64_t launches = cdiv(H, std::min(fit, H));
+  return cdiv(cdiv(H, launches), group) * group;
+}
+
 // paged.choose_launch: workgroups of the balanced launch, 0 = one workgroup per (sequence, kv head) pair
 int balanced_workgroups(int64_t seqs, int64_t Hkv, int64_t group, int64_t D, int64_t max_context, int cus) {
   const int wgs = cus * (D <= 128 ? 2 : 1);
@@ -364,7 +370,7 @@ variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, 
   int bn = B, hn = H;   // batch entries and heads per launch
   Tensor ds;
   if (heads >= (int64_t)B * H) ds = ds_workspace(q, B, H, M, N, 1);
-  else if (heads > 0) ds = ds_workspace(q, bn = 1, hn = (int)std::min<int64_t>(heads, H), M, N, 1);
+  else if (heads > 0) ds = ds_workspace(q, bn = 1, hn = (int)even_heads(heads, H, group), M, N, 1);
   if (!ds.defined()) { bn = B; hn = H; }
 
   // Slices of dK / dV: one per `chunk` query heads (the kernels that sum query heads are built without dropout) and
@@ -601,7 +607,7 @@ struct PiecewiseNode : torch::autograd::Function<PiecewiseNode> {
     Tensor ds;
     int64_t nb = B, step = H;   // batch entries and heads per launch
     if (heads >= (int64_t)B * H) ds = ds_workspace(q1, B, H, M, N, 2);
-    else if (heads > 0) ds = ds_workspace(q1, nb = 1, step = std::min<int64_t>(heads, H), M, N, 2);
+    else if (heads > 0) ds = ds_workspace(q1, nb = 1, step = even_heads(heads, H, 1), M, N, 2);
     if (!ds.defined()) { nb = B; step = H; }
     for (int64_t b = 0; b < B; b += nb)
       for (int64_t h0 = 0; h0 < H; h0 += step) {

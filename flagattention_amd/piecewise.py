@@ -9,7 +9,7 @@ import math
 import torch
 
 from . import _abi, _config, _lib, flash
-from .flash import NothingToAttend, _ds_workspace, ds_heads_per_launch
+from .flash import NothingToAttend, _ds_workspace, ds_heads_per_launch, even_heads
 
 __all__ = ["attention"]
 
@@ -84,7 +84,7 @@ class PiecewiseAttention(torch.autograd.Function):
             if heads >= B * H:
                 ds = _ds_workspace(lib, q1.device, B, H, M, N, grids=2)
             elif heads > 0:
-                heads = min(heads, H)
+                heads = even_heads(heads, H, 1)
                 ds = _ds_workspace(lib, q1.device, 1, heads, M, N, grids=2)
             if ds is None:   # dS not worth keeping for this shape, or no memory for it: recompute it
                 _abi.pw_bwd_dkdv(lib, q1, k1, q2, k2, v, do, L, delta, dk1, dk2, dv, *args)
