@@ -1,9 +1,11 @@
 """Loader for the C-ABI kernel library (``libflagattn_hip.so``, declared in ``include/flagattn.h``).
 
-There is no fallback: if the library has not been built, or cannot be loaded, every operator raises.
+There is no fallback for the kernels: if the library has not been built, or cannot be loaded, every operator raises.
 """
 import ctypes
 import os
+import sys
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libflagattn_hip.so"
@@ -94,21 +96,33 @@ def get():
     return _lib
 
 
+class PythonForm:
+    """Stands in for the native host path where that cannot be loaded: it takes no call, so each operator runs the Python
+    form of the same host logic on the same kernels."""
+
+    @staticmethod
+    def _not_taken(*args):
+        return NotImplemented
+
+    flash = piecewise = paged = _not_taken
+
+
 _native = None
 
 
 def native():
-    """The native host path of the operators for GPU tensors (``_host.so``, built with the kernel library from
-    ``csrc/host.cpp``); raises if it is not there."""
+    """The native host path of the operators for GPU tensors (``_host.so``, built from ``csrc/host.cpp`` against one
+    interpreter and one torch).  Where it is missing or does not load, the reason is reported once and ``PythonForm`` is
+    returned: short calls are then slower (a decode step 38 us instead of 11), results are the same."""
     global _native
     if _native is None:
         get()
         try:
-            from . import _host
-        except ImportError as e:
-            raise RuntimeError("_host.so is not built for this interpreter and torch; build it with "
-                               "`make -C flagattention_amd/csrc` -- there is no fallback implementation") from e
-        from . import _abi, flash, piecewise
-        _host.bind(_abi.check, flash.backward_settings, piecewise.backward_settings)
-        _native = _host
+            from . import _abi, _host, flash, piecewise
+            _host.bind(_abi.check, flash.backward_settings, piecewise.backward_settings)
+            _native = _host
+        except (ImportError, OSError) as e:
+            warnings.warn(f"the native host path is not used, calls are prepared in Python: {e} (build it with "
+                          f"`make -C flagattention_amd/csrc host PYTHON={sys.executable}`)", RuntimeWarning, stacklevel=3)
+            _native = PythonForm
     return _native

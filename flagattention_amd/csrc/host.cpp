@@ -773,4 +773,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__host(void) {
+  if (fa_version() != FA_ABI_VERSION)   // the two are built apart
+    return PyErr_Format(PyExc_ImportError, "_host.so was built for revision %d of the C interface, the kernel library is revision %d",
+                        FA_ABI_VERSION, fa_version());
+  return PyModule_Create(&kModule);
+}
