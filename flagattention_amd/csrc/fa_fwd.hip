@@ -274,9 +274,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
     for (; it < t_end; ++it) { step(std::false_type{}, it, t_end, stage); stage ^= 1; }
   }
 
-  // ---- epilogue: O = acc / l, L = m * scale + ln(l); rows that saw no key give O = 0, L = -inf ----
+  // ---- epilogue: O = acc / l, L = m * scale + ln(l); rows that saw no key give O = 0, L = -inf (a sum that is NaN is
+  //      not one of them: O and L become NaN, and the merge of pieces cannot take the piece for an empty one) ----
   const float l_tot = l_i + hw::xor32(l_i);
-  const bool empty = !(l_tot > 0.f);
+  const bool empty = l_tot == 0.f;
   const float inv = empty ? 0.f : (DROP ? 1.f / ((1.f - p.dropout_p) * l_tot) : 1.f / l_tot);
   if (!(PW || DROP) && p.num_splits > 0) {
     if (my_m >= M) return;

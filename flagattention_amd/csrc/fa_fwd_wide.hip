@@ -483,12 +483,13 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 1) fa_fwd_wide_kernel(FwdParams p) {
     static_for<8>([&](auto t) { hw::pinned_o_clear<decltype(t)::value>(O); });
   }
 
-  // ---- epilogue: O = acc / l, L = m * scale + ln(l); rows that saw no key give O = 0, L = -inf ----
+  // ---- epilogue: O = acc / l, L = m * scale + ln(l); rows that saw no key give O = 0, L = -inf (a sum that is NaN
+  //      is not one of them) ----
   static_for<2>([&](auto x_tag) {
     constexpr int x = decltype(x_tag)::value;
     const float l_lane = lsum[x][0] + lsum[x][1];
     const float l_tot = l_lane + hw::xor32(l_lane);
-    const bool empty = !(l_tot > 0.f);
+    const bool empty = l_tot == 0.f;
     const float inv = empty ? 0.f : 1.f / l_tot;
     if (my_m[x] < M) {
       const bool whole = p.num_splits <= 0;

@@ -6,7 +6,8 @@
 // share that kv head, so the keys and values of a split are read once for the whole GQA group.
 // Partial outputs are fp16 whatever the input dtype, as in the reference (flash.py:96); a split
 // that holds no visible key for a row stores 0 and a log-normalizer of -inf, and the merge weights
-// by select so that such splits drop out instead of producing NaN.
+// by select so that such splits drop out instead of producing NaN.  A NaN in a split's row sum goes to both and
+// through the merge into the result.
 #include "decode.hpp"
 #include "params.hpp"
 
@@ -71,7 +72,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_splitkv_kernel(SplitParams p) {
     if (r < rows) {
       const int g = r / M, m = r % M;
       const int64_t slot = (((int64_t)batch * p.H + hk * p.group + g) * p.num_splits + split) * M + m;
-      const bool empty = !(res.row_sum[e] > 0.f);
+      const bool empty = res.row_sum[e] == 0.f;
       ((hw::half_t*)p.part_o)[slot * D + d] = (hw::half_t)(empty ? 0.f : res.o[e] / res.row_sum[e]);
       if (d == 0)
         p.part_lse[slot] = empty ? neg_inf() : res.row_max[e] * p.sm_scale + hw::log_nat(res.row_sum[e]);
@@ -157,7 +158,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_combine_kernel(CombineParams p) {
     if (group > 0) return;
   }
   if (my_row >= total_rows) return;
-  const float inv = z > 0.f ? 1.f / z : 0.f;
+  const float inv = z == 0.f ? 0.f : 1.f / z;   // z is NaN where a piece's log-normalizer is
   const int b = (int)(bh / p.H), h = (int)(bh % p.H);
   T* o = (T*)p.o.ptr + b * p.o.sb + h * p.o.sh + (int64_t)m * p.o.st + col;
   u32x4 w;
@@ -165,7 +166,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) fa_combine_kernel(CombineParams p) {
   for (int e = 0; e < 4; ++e)
     w[e] = (uint32_t)hw::bits16<T>(acc[2 * e] * inv) | ((uint32_t)hw::bits16<T>(acc[2 * e + 1] * inv) << 16);
   *(u32x4*)o = w;
-  if (col == 0) p.lse[row] = z > 0.f ? top + hw::log_nat(z) : neg_inf();
+  if (col == 0) p.lse[row] = z == 0.f ? neg_inf() : top + hw::log_nat(z);
 }
 
 template <class T, bool UNIFORM>

@@ -138,7 +138,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (D <= 128 ? 2 : 1)) paged_attn_kernel
     const int row = idx / D, d = idx % D;
     const int g = rb * 16 + row;
     if (g < G) {
-      const float val = res.row_sum[e] > 0.f ? res.o[e] / res.row_sum[e] : 0.f;
+      const float val = res.row_sum[e] == 0.f ? 0.f : res.o[e] / res.row_sum[e];
       if (p.partition_size > 0) {
         const int64_t slot = (((int64_t)seq * p.Hkv + hk) * p.num_parts + part) * G + g;
         ((T*)p.tmp_out)[slot * D + d] = (T)val;
@@ -154,7 +154,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (D <= 128 ? 2 : 1)) paged_attn_kernel
 }
 
 // out = sum_j w_j o_j / sum_j w_j with w_j = l_j exp(m_j - max_j m_j) over n partial results of one
-// output element.  The loads of eight partials are issued together: a loop that loads, waits and
+// output element; partials of sum 0 (no visible key) drop out, a sum that is NaN makes the result NaN.  The loads of eight partials are issued together: a loop that loads, waits and
 // accumulates one partial at a time costs a full memory latency per partial.
 template <class FM, class FL, class FO>
 FA_DEVICE float merge_partials(int n, FM m_of, FL l_of, FO o_of) {
@@ -179,14 +179,14 @@ FA_DEVICE float merge_partials(int n, FM m_of, FL l_of, FO o_of) {
     }
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      if (j0 + u < n && lv[u] > 0.f) {
+      if (j0 + u < n && lv[u] != 0.f) {
         const float wgt = lv[u] * hw::exp2_fast((mv[u] - top) * kLog2e);
         z += wgt;
         acc += wgt * ov[u];
       }
     }
   }
-  return z > 0.f ? acc / z : 0.f;
+  return z == 0.f ? 0.f : acc / z;
 }
 
 // One workgroup per (sequence, kv head): out = sum_p tmp_out_p * w_p / sum_p w_p with
@@ -338,7 +338,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (D <= 128 ? 2 : 1)) paged_balanced_ke
       const int row = idx / D, d = idx % D;
       const int g = rb * 16 + row;
       if (idx < 16 * D && g < G) {
-        const float val = res.row_sum[e] > 0.f ? res.o[e] / res.row_sum[e] : 0.f;
+        const float val = res.row_sum[e] == 0.f ? 0.f : res.o[e] / res.row_sum[e];
         if (whole) {
           ((T*)p.out)[(int64_t)seq * p.o_ss + (int64_t)(hk * G + g) * p.o_sh + d] = (T)val;
         } else {
@@ -411,7 +411,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) paged_balanced_reduce_kernel(PagedPara
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
-        if (j0 + u < n && lv[u] > 0.f) {
+        if (j0 + u < n && lv[u] != 0.f) {
           const float wgt = lv[u] * hw::exp2_fast((mv[u] - top) * kLog2e);
           z += wgt;
 #pragma unroll
@@ -429,9 +429,10 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) paged_balanced_reduce_kernel(PagedPara
       if (share == 0) {
         for (int g = 1; g < shares; ++g) top = fmaxf(top, area[5 * kThreads + tid + g * side * kLanes]);
         float sum[4] = {0.f, 0.f, 0.f, 0.f}, zs = 0.f;
-        for (int g = 0; g < shares && top > neg_inf(); ++g) {
+        for (int g = 0; g < shares; ++g) {
           const int at = tid + g * side * kLanes;
-          const float wgt = hw::exp2_fast((area[5 * kThreads + at] - top) * kLog2e);
+          const float own = area[5 * kThreads + at];   // -inf in all shares: nothing but zeroes, or NaN, to add
+          const float wgt = own == top ? 1.f : hw::exp2_fast((own - top) * kLog2e);
           zs += wgt * area[4 * kThreads + at];
 #pragma unroll
           for (int e = 0; e < 4; ++e) sum[e] += wgt * area[e * kThreads + at];
@@ -442,7 +443,7 @@ FA_KERNEL void FA_LAUNCH_BOUNDS(kThreads) paged_balanced_reduce_kernel(PagedPara
       }
     }
     if (share == 0 && row < rows) {
-      const float inv = z > 0.f ? 1.f / z : 0.f;
+      const float inv = z == 0.f ? 0.f : 1.f / z;
       T* o = (T*)p.out + (int64_t)seq * p.o_ss + (int64_t)(hk * G + rb * 16 + row) * p.o_sh + d;
       if (out_aligned) {
         hw::u32x2 packed;
