@@ -7,6 +7,7 @@
 //     block and the half h = l / 32 selects which rows / which 8 of the 16 contraction indices.
 #pragma once
 #include <atomic>
+#include <initializer_list>
 #include <mutex>
 #include <type_traits>
 #include <unordered_map>
@@ -308,6 +309,15 @@ int launch(void (*kern)(P), dim3 grid, size_t lds_bytes, hipStream_t stream, con
   }
   hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, stream, p);
   return (int)hipGetLastError();
+}
+
+// Workgroups of a 1-D launch (the product of the factors), 0 if there are more than a grid can hold.  Formed in 64 bits and
+// compared factor by factor: a product of ints that wraps would launch part of the tiles, or none, without an error.
+inline unsigned workgroups(std::initializer_list<int64_t> factors) {
+  int64_t n = 1;
+  for (int64_t f : factors)
+    if ((n *= f) > 0x7fffffff) return 0;
+  return (unsigned)n;
 }
 
 // Workgroups of a kernel that a compute unit of the current device holds; asked once per kernel and device.

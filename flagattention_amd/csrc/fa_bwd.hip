@@ -1217,7 +1217,8 @@ int run_sum_slices(const SumParams& p, hipStream_t stream) {
 template <class T, bool PW, bool DS, int DROP, bool GROUPED>
 static int launch_dkdv(const BwdParams& p, hipStream_t stream) {
   const int chunk = GROUPED ? (p.chunk > 0 ? p.chunk : p.group) : 1;
-  dim3 grid(((p.N + 127) / 128) * (p.H / chunk) * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
+  const dim3 grid(workgroups({((int64_t)p.N + 127) / 128, p.H / chunk, p.B, p.pieces > 0 ? p.pieces : 1}));
+  if (!grid.x) return kBadArgument;
   switch (p.D) {
     case 16: return launch_dealt(fa_bwd_dkdv_kernel<T, 16, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 16, PW, DROP>::LDS_BYTES, stream, p);
     case 32: return launch_dealt(fa_bwd_dkdv_kernel<T, 32, PW, DS, DROP, GROUPED>, grid, KvCfg<T, 32, PW, DROP>::LDS_BYTES, stream, p);
@@ -1229,7 +1230,8 @@ static int launch_dkdv(const BwdParams& p, hipStream_t stream) {
 
 template <class T, bool PW, int DROP>
 static int launch_dq(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
+  const dim3 grid(workgroups({((int64_t)p.M + 127) / 128, p.H, p.B, p.pieces > 0 ? p.pieces : 1}));
+  if (!grid.x) return kBadArgument;
   switch (p.D) {
     case 16: return launch_dealt(fa_bwd_dq_kernel<T, 16, PW, DROP>, grid, QCfg<T, 16, PW>::LDS_BYTES, stream, p);
     case 32: return launch_dealt(fa_bwd_dq_kernel<T, 32, PW, DROP>, grid, QCfg<T, 32, PW>::LDS_BYTES, stream, p);
@@ -1296,7 +1298,8 @@ int run_bwd_dq(const BwdParams& a, bool piecewise, hipStream_t stream) {
 
 template <class T, bool PW>
 static int launch_dq_from_ds(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.pieces > 0 ? p.pieces : 1), 1, 1);
+  const dim3 grid(workgroups({((int64_t)p.M + 127) / 128, p.H, p.B, p.pieces > 0 ? p.pieces : 1}));
+  if (!grid.x) return kBadArgument;
   switch (p.D) {
     case 16: return launch_dealt(fa_bwd_dq_from_ds_kernel<T, 16, PW>, grid, QdsCfg<T, 16>::LDS_BYTES, stream, p);
     case 32: return launch_dealt(fa_bwd_dq_from_ds_kernel<T, 32, PW>, grid, QdsCfg<T, 32>::LDS_BYTES, stream, p);

@@ -315,7 +315,8 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, (FwdCfg<T, D, PW>::WAVES_PER_SIMD)) f
 
 template <class T, bool PW, bool DROP>
 static int launch_fwd(const FwdParams& p, hipStream_t stream) {
-  dim3 grid(((p.M + 127) / 128) * p.H * p.B * (p.num_splits > 0 ? p.num_splits : 1), 1, 1);
+  const dim3 grid(workgroups({((int64_t)p.M + 127) / 128, p.H, p.B, p.num_splits > 0 ? p.num_splits : 1}));
+  if (!grid.x) return kBadArgument;
   switch (p.D) {
     case 16: return launch_dealt(fa_fwd_kernel<T, 16, PW, DROP>, grid, FwdCfg<T, 16, PW>::LDS_BYTES, stream, p);
     case 32: return launch_dealt(fa_fwd_kernel<T, 32, PW, DROP>, grid, FwdCfg<T, 32, PW>::LDS_BYTES, stream, p);

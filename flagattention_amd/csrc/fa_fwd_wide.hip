@@ -525,8 +525,8 @@ bool fwd_wide_supported(const FwdParams& p) {
 int run_fwd_wide(const FwdParams& p, hipStream_t stream) {
   if (p.B <= 0 || p.H <= 0 || p.M <= 0 || p.N < 0 || p.group <= 0 || !fwd_wide_supported(p)) return kBadArgument;
   if (p.num_splits < 0 || (p.num_splits > 0 && (p.split_size <= 0 || !p.part_o || !p.part_lse))) return kBadArgument;
-  const int pieces = p.num_splits > 0 ? p.num_splits : 1;
-  dim3 grid(((p.M + WideCfg::BM - 1) / WideCfg::BM) * p.H * p.B * pieces, 1, 1);
+  const dim3 grid(workgroups({((int64_t)p.M + WideCfg::BM - 1) / WideCfg::BM, p.H, p.B, p.num_splits > 0 ? p.num_splits : 1}));
+  if (!grid.x) return kBadArgument;
   if (p.dtype == kDtypeF16) return launch(fa_fwd_wide_kernel<hw::half_t>, grid, WideCfg::LDS_BYTES, stream, p);
   if (p.dtype == kDtypeBF16) return launch(fa_fwd_wide_kernel<hw::bf16_t>, grid, WideCfg::LDS_BYTES, stream, p);
   return kUnsupported;

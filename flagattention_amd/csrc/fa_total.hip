@@ -119,7 +119,8 @@ FA_KERNEL void FA_LAUNCH_BOUNDS2(kThreads, 2) fa_total_kernel(TotalParams p) {
 
 template <class T>
 static int launch_total(const TotalParams& p, hipStream_t stream) {
-  dim3 grid(((p.N + 127) / 128) * p.H * p.B, 1, 1);
+  const dim3 grid(workgroups({((int64_t)p.N + 127) / 128, p.H, p.B}));
+  if (!grid.x) return kBadArgument;
   switch (p.D) {
     case 16: return launch_dealt(fa_total_kernel<T, 16>, grid, TotCfg<T, 16>::LDS_BYTES, stream, p);
     case 32: return launch_dealt(fa_total_kernel<T, 32>, grid, TotCfg<T, 32>::LDS_BYTES, stream, p);

@@ -1,11 +1,13 @@
 """The C-ABI library loads without a GPU and exports exactly what include/flagattn.h declares;
 the ctypes signature table matches the header's argument counts.  No compute calls."""
+import ctypes
 import os
 import re
 
 import pytest
 
 from flagattention_amd import _lib
+from tests.sim import simlib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "flagattn.h")
@@ -95,3 +97,25 @@ def test_integration_doc_binding_matches_signature_table():
         depth -= ch in ")]"
         nargs += (ch == "," and depth == 0)
     assert nargs == len(table)
+
+
+@pytest.mark.parametrize("entry", ["dkdv", "dkdv_ds", "dq", "dq_from_ds", "fwd", "total"])
+def test_launches_of_more_workgroups_than_a_grid_holds_are_refused(entry):
+    """2^32 workgroups: as a product of ints that is a grid of none, which would return success with nothing written.
+    (Nothing may be launched here, so no tensor behind the pointers has these sizes.)"""
+    lib = simlib.get()
+    memory = ctypes.create_string_buffer(4096 + 16)
+    at = (ctypes.addressof(memory) + 15) & ~15
+    view, ptr = ctypes.byref(_lib.View4(at, 0, 0, 0)), ctypes.c_void_p(at)
+    B, H, T, D, scale = 256, 256, 128 * 1024, 64, ctypes.c_float(0.125)     # 2^10 tiles, and 64 pieces
+    kind, size, enough = 1 | (64 << 8), (B, H, H, T, T, D), 1 << 62
+    calls = {
+        "dkdv": lambda: lib.fa_bwd_dkdv(kind, view, view, view, view, ptr, ptr, view, view, 1, *size, 0, scale, 0.0, 0, 0, None),
+        "dkdv_ds": lambda: lib.fa_bwd_dkdv_ds(kind, view, view, view, view, ptr, ptr, view, view, 1, ptr, enough, *size, 0, scale,
+                                              0.0, 0, 0, None),
+        "dq": lambda: lib.fa_bwd_dq(kind, view, view, view, view, ptr, ptr, view, *size, 0, scale, 0.0, 0, 0, None),
+        "dq_from_ds": lambda: lib.fa_bwd_dq_from_ds(kind, view, ptr, enough, view, *size, 0, scale, None),
+        "fwd": lambda: lib.fa_fwd(1, view, view, view, view, ptr, 64 * B, H, H, T, T, D, 0, scale, 0.0, 0, 0, 128, None),
+        "total": lambda: lib.fa_total_attn(1, view, view, ptr, ptr, 64 * B, H, H, T, T, D, 0, scale, None),
+    }
+    assert calls[entry]() == -1
