@@ -686,6 +686,7 @@ PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!THPVariable_Check(a[i])) return not_taken();
   const Tensor &q = THPVariable_Unpack(a[0]), &kc = THPVariable_Unpack(a[1]), &vc = THPVariable_Unpack(a[2]),
                &lens = THPVariable_Unpack(a[3]), &bt = THPVariable_Unpack(a[4]);
+  if (!plain_call({&q, &kc, &vc, &lens, &bt})) return not_taken();
   if (!q.is_cuda() || q.dim() != 3 || q.layout() != at::kStrided || !is_operand(kc, kc) || !is_operand(vc, kc) ||
       kc.device() != q.device() || kc.scalar_type() != q.scalar_type() || !type_ok(q))
     return not_taken();

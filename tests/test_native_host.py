@@ -159,3 +159,36 @@ def test_transforms_and_tracers_see_a_python_function(op):
         a, b = outcome(lambda: form(native)), outcome(lambda: form(python))
         assert isinstance(a, torch.Tensor) == isinstance(b, torch.Tensor), (a, b)
         assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a is b, (a, b)
+
+
+def paged_arguments():
+    lens, table = torch.tensor([40, 9], dtype=torch.int32, device="cuda"), torch.arange(6, device="cuda").reshape(2, 3)
+    return randn(1, 2, 4, 64)[0], randn(6, 4, 16, 64), randn(6, 4, 16, 64), lens, table
+
+
+@pytest.mark.gpu
+def test_paged_call_is_made_in_python_where_something_listens():
+    """As for the other operators: the native path launches past the dispatcher, so it takes no call that a dispatch mode, a
+    tracer, a transform or a tangent should see."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    q, *rest = paged_arguments()
+
+    def native(query):
+        return _lib.native().paged(query, *rest, 0.125, 40)
+
+    class Recorder(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    assert isinstance(native(q), torch.Tensor)
+    seen, answers = [], []
+    with Recorder():
+        flag_attn.paged_attention(q, *rest, 0.125, 40)
+    assert any("empty" in name for name in seen)
+    with forward_ad.dual_level():
+        answers.append(native(forward_ad.make_dual(q, torch.ones_like(q))))
+    torch.vmap(lambda query: answers.append(native(query)) or query)(torch.stack([q, q]))
+    torch.jit.trace(lambda query: answers.append(native(query)) or query, (q,), check_trace=False)
+    assert len(answers) == 3 and all(a is NotImplemented for a in answers)
