@@ -501,11 +501,18 @@ bool needs_grad(std::initializer_list<const Tensor*> ts) {
 
 PyObject* not_taken() { Py_RETURN_NOTIMPLEMENTED; }
 
+// Tensors and parameters.  A subclass of either gets its own type back from the Python form's torch.empty_like.
+bool plain_tensors(PyObject* const* a, int n) {
+  for (int i = 0; i < n; ++i)
+    if (!THPVariable_CheckExact(a[i])) return false;
+  return true;
+}
+
 // flash(q, k, v, causal, sm_scale or None, dropout_p, return_log_normalizer, return_total_attention, return_seed_offset)
 PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK(n == 9, "flash: nine arguments");
-  if (!THPVariable_Check(a[0]) || !THPVariable_Check(a[1]) || !THPVariable_Check(a[2])) return not_taken();
+  if (!plain_tensors(a, 3)) return not_taken();
   const Tensor &q = THPVariable_Unpack(a[0]), &k = THPVariable_Unpack(a[1]), &v = THPVariable_Unpack(a[2]);
   FlashCall c = {};
   const int causal = PyObject_IsTrue(a[3]), want_lse = PyObject_IsTrue(a[6]), want_total = PyObject_IsTrue(a[7]),
@@ -637,8 +644,7 @@ struct PiecewiseNode : torch::autograd::Function<PiecewiseNode> {
 PyObject* piecewise(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK(n == 8, "piecewise: eight arguments");
-  for (int i = 0; i < 5; ++i)
-    if (!THPVariable_Check(a[i])) return not_taken();
+  if (!plain_tensors(a, 5)) return not_taken();
   const Tensor &q1 = THPVariable_Unpack(a[0]), &k1 = THPVariable_Unpack(a[1]), &q2 = THPVariable_Unpack(a[2]),
                &k2 = THPVariable_Unpack(a[3]), &v = THPVariable_Unpack(a[4]);
   if (!plain_call({&q1, &k1, &q2, &k2, &v})) return not_taken();
@@ -682,8 +688,7 @@ bool row_ready(const Tensor& t) {   // a (num_seqs, heads, D) tensor the kernels
 PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK(n == 7, "paged: seven arguments");
-  for (int i = 0; i < 5; ++i)
-    if (!THPVariable_Check(a[i])) return not_taken();
+  if (!plain_tensors(a, 5)) return not_taken();
   const Tensor &q = THPVariable_Unpack(a[0]), &kc = THPVariable_Unpack(a[1]), &vc = THPVariable_Unpack(a[2]),
                &lens = THPVariable_Unpack(a[3]), &bt = THPVariable_Unpack(a[4]);
   if (!plain_call({&q, &kc, &vc, &lens, &bt})) return not_taken();

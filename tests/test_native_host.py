@@ -192,3 +192,23 @@ def test_paged_call_is_made_in_python_where_something_listens():
     torch.vmap(lambda query: answers.append(native(query)) or query)(torch.stack([q, q]))
     torch.jit.trace(lambda query: answers.append(native(query)) or query, (q,), check_trace=False)
     assert len(answers) == 3 and all(a is NotImplemented for a in answers)
+
+
+@pytest.mark.gpu
+def test_tensor_subclasses_get_their_own_type_back():
+    """A subclass without __torch_dispatch__ is what the Python form's torch.empty_like makes of it; parameters are taken as
+    the tensors they are."""
+    class Named(torch.Tensor):
+        pass
+
+    q, k, v, q2, k2 = (randn(1, 4, 96, 64) for _ in range(5))
+    query, *rest = paged_arguments()
+    for kind in (Named, torch.nn.Parameter):
+        own = (lambda t: t.as_subclass(Named)) if kind is Named else torch.nn.Parameter
+        outs = [flag_attn.flash_attention(own(q), k, v), flag_attn.piecewise_attention(own(q), k, q2, k2, v, 40),
+                flag_attn.paged_attention(own(query), *rest, 0.125, 40)]
+        assert [type(o) for o in outs] == [Named if kind is Named else torch.Tensor] * 3
+        assert [o.requires_grad for o in outs] == [kind is not Named] * 2 + [False]
+    plain = flag_attn.flash_attention(q, k, v), flag_attn.piecewise_attention(q, k, q2, k2, v, 40), flag_attn.paged_attention(query, *rest, 0.125, 40)
+    for a, b in zip(outs, plain):
+        assert torch.equal(a, b)
