@@ -5,11 +5,13 @@
 // longer than they do -- 38 us for a decode step, 20 us for a paged one, 195 us for a forward and backward over
 // 512 tokens (of 42 us of kernels).
 //
-// The Python modules hold the reference form of every decision made here (`flash.py`, `split_kv.py`, `paged.py`,
-// `piecewise.py`).  It runs whenever a tile-config hook has been replaced, for tensors that are not on a GPU, and
-// for every call this file does not take (it then answers NotImplemented, before any effect); arguments that are
-// in error are among those, so that their messages have one source.  `decisions()` exposes the numbers chosen here
-// to the test that compares them with the Python functions.
+// The Python modules hold the reference form of the launch decisions made here (`flash.py`, `split_kv.py`, `paged.py`,
+// `piecewise.py`).  It runs whenever a tile-config hook has been replaced, for tensors that are not on a GPU, where
+// this extension is not built, and for every call this file does not take (it then answers NotImplemented, before any
+// effect); arguments that are in error are among those, so that their messages have one source.  `decisions()` and the
+// functions after it expose the numbers chosen here to the tests that compare them with the Python functions.  One
+// decision is made only here: whether a dropout mask is kept for the backward (`keeps_mask`); the Python form always
+// draws it again, with the same result.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -125,14 +127,11 @@ int dkdv_heads_per_slice(int64_t B, int64_t H, int group, int64_t N, int cus) {
   return 1;
 }
 
-// How a backward kernel's workgroups use a compute unit: `slots` of them share it; a step (64 queries or keys) takes one
-// `alone` us, each of a full set `shared` us, and what comes before and behind the steps `around` us.  Measured on long
-// launches (shared) and on launches of less than one workgroup per unit (alone).
+// flash._DKDV_128 and those after it: how a backward kernel's workgroups use a compute unit (what is measured stands there)
 struct Pace { int slots; double alone, shared, around; };
 constexpr Pace kDkdv128 = {1, 1.7, 2.1, 6.0}, kDkdv64 = {2, 1.05, 2.1, 5.0}, kDq = {2, 1.1, 1.6, 4.0}, kDqFromDs = {2, 1.15, 1.6, 4.0};
 
-// Estimated us of a launch of `tiles` result tiles of up to `steps` steps each, every tile's sum dealt to `pieces`
-// workgroups.  Under the causal mask workgroups start longest first and average half the longest.
+// flash._launch_us
 double launch_us(const Pace& pace, int64_t tiles, double steps, bool causal, int pieces, double slice_bytes, int cus) {
   const double wgs = (double)tiles * pieces, per = steps / pieces, full = (double)cus * pace.slots;
   double t;
@@ -145,8 +144,7 @@ double launch_us(const Pace& pace, int64_t tiles, double steps, bool causal, int
   t += pace.around * std::max(1.0, wgs / full);
   return pieces == 1 ? t : t + 3.0 + 2 * wgs * slice_bytes / 5e6;   // fp32 slices written and read back at 5 TB/s, and the launch that adds them
 }
-// Workgroups that share the sum of one result tile (FA_PIECES): more than one where a launch is as long as its longest
-// workgroup, or its last round of workgroups is nearly empty, and that costs more than adding the pieces does.
+// flash._contraction_pieces
 int contraction_pieces(const Pace& pace, int64_t tiles, int64_t steps, bool causal, double slice_bytes, int cus) {
   int best = 1;
   double least = launch_us(pace, tiles, (double)steps, causal, 1, slice_bytes, cus);
@@ -155,6 +153,13 @@ int contraction_pieces(const Pace& pace, int64_t tiles, int64_t steps, bool caus
     if (t < 0.95 * least) { best = n; least = t; }
   }
   return best;
+}
+
+// flash.gradient_pieces: of dK and dV, of dQ
+struct GradientPieces { int kv, q; };
+GradientPieces gradient_pieces(int64_t B, int64_t H, int64_t M, int64_t N, int64_t D, bool causal, int chunk, bool ds_kept, int cus) {
+  return {chunk > 1 ? 1 : contraction_pieces(D == 128 ? kDkdv128 : kDkdv64, cdiv(N, 128) * B * H, cdiv(M, 64), causal, 2 * 4.0 * 128 * D, cus),
+          contraction_pieces(ds_kept ? kDqFromDs : kDq, cdiv(M, 128) * B * H, cdiv(N, 64), causal, 4.0 * 128 * D, cus)};
 }
 
 // flash.ds_heads_per_launch
@@ -376,9 +381,7 @@ variable_list flash_backward(const Tensor& q, const Tensor& k, const Tensor& v, 
   // Slices of dK / dV: one per `chunk` query heads (the kernels that sum query heads are built without dropout) and
   // piece of the query axis; of dQ: one per piece of the key axis.  More than one per result: fp32, added at the end.
   int chunk = c.dropout_p > 0 ? 1 : dkdv_heads_per_slice(bn, hn, group, N, cus);
-  // (counted over all heads, so that launches in turns add up in the same order as one launch)
-  int kv_pieces = chunk > 1 ? 1 : contraction_pieces(D == 128 ? kDkdv128 : kDkdv64, cdiv(N, 128) * B * H, cdiv(M, 64), c.causal, 2 * 4.0 * 128 * D, cus);
-  int q_pieces = contraction_pieces(ds.defined() ? kDqFromDs : kDq, cdiv(M, 128) * B * H, cdiv(N, 64), c.causal, 4.0 * 128 * D, cus);
+  auto [kv_pieces, q_pieces] = gradient_pieces(B, H, M, N, D, c.causal, chunk, ds.defined(), cus);
   int kv_slices = group / chunk * kv_pieces;   // per kv head
   Tensor dk = empty({B, Hk, N, D}, k.scalar_type(), q), dv = empty({B, Hk, N, D}, k.scalar_type(), q);
   Tensor dq = empty({B, H, M, D}, q.scalar_type(), q), dk_s = dk, dv_s = dv, dq_s = dq;
@@ -760,6 +763,22 @@ PyObject* pieces_of_forward(PyObject*, PyObject* args) {
   return PyLong_FromLong(forward_pieces(B, H, Hk, M, N, D, split, (int)cus));
 }
 
+// gradient_pieces(B, H, M, N, D, causal, chunk, ds_kept, num_cus) -> (dK/dV, dQ)
+PyObject* pieces_of_gradients(PyObject*, PyObject* args) {
+  long long B, H, M, N, D, cus;
+  int causal, chunk, ds_kept;
+  if (!PyArg_ParseTuple(args, "LLLLLpipL", &B, &H, &M, &N, &D, &causal, &chunk, &ds_kept, &cus)) return nullptr;
+  const GradientPieces p = gradient_pieces(B, H, M, N, D, causal, chunk, ds_kept, (int)cus);
+  return Py_BuildValue("(ii)", p.kv, p.q);
+}
+
+// keeps_mask(N, D)
+PyObject* mask_is_kept(PyObject*, PyObject* args) {
+  long long N, D;
+  if (!PyArg_ParseTuple(args, "LL", &N, &D)) return nullptr;
+  return PyBool_FromLong(keeps_mask(N, D));
+}
+
 // bind(abi.check, flash settings, piecewise settings)
 PyObject* bind(PyObject*, PyObject* args) {
   if (!PyArg_ParseTuple(args, "OOO", &g_check, &g_flash_settings, &g_piecewise_settings)) return nullptr;
@@ -773,6 +792,8 @@ PyMethodDef kMethods[] = {
     {"paged", (PyCFunction)(void*)paged, METH_FASTCALL, nullptr},
     {"decisions", decisions, METH_VARARGS, nullptr},
     {"forward_pieces", pieces_of_forward, METH_VARARGS, nullptr},
+    {"gradient_pieces", pieces_of_gradients, METH_VARARGS, nullptr},
+    {"keeps_mask", mask_is_kept, METH_VARARGS, nullptr},
     {"bind", bind, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

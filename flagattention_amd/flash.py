@@ -258,41 +258,50 @@ class FlashAttention(torch.autograd.Function):
             elif heads > 0:
                 heads = even_heads(heads, H, group)
                 ds = _ds_workspace(lib, q.device, 1, heads, M, N)
+            # launches of all heads, or (bounded workspace) of one batch entry and `hn` heads at a time
+            bn, hn = (1, heads) if ds is not None and heads < B * H else (B, H)
             # dK/dV come out summed over each kv head's group of query heads (flash.py:205-206,250-251
-            # of the reference produce one slice per query head and reduce afterwards), or over chunks of
-            # it, then as fp32 slices that are added below
-            # the kernels that sum query heads are built without dropout
-            in_turns = ds is not None and heads < B * H     # launches of one batch entry and `heads` heads
-            chunk = 1 if dropout[0] > 0 else dkdv_heads_per_slice(1 if in_turns else B, heads if in_turns else H,
-                                                                  group, N, _num_cus())
-            slices = H // chunk
-            pieces = 1 if slices > Hk else 0
-            dk = torch.empty((B, slices, N, D), dtype=torch.float32 if pieces else k.dtype, device=q.device)
-            dv = torch.empty((B, slices, N, D), dtype=torch.float32 if pieces else v.dtype, device=q.device)
+            # of the reference produce one slice per query head and reduce afterwards), or over chunks of it;
+            # the kernels that sum query heads are built without dropout.  A sum may be dealt to several
+            # workgroups as well; what is not one sum per result leaves fp32 slices that are added at the end.
+            chunk = 1 if dropout[0] > 0 else dkdv_heads_per_slice(bn, hn, group, N, _num_cus())
+            # (not with replaced tile hooks: launches of any size then add up in the order that the tiles give)
+            kv_pieces, q_pieces = (1, 1) if _hooks_replaced() else \
+                gradient_pieces(B, H, M, N, D, causal, chunk, ds is not None, _num_cus())
+            kv_slices = group // chunk * kv_pieces   # per kv head
+            dk, dv = (torch.empty((B, Hk, N, D), dtype=k.dtype, device=q.device) for _ in range(2))
             dq = torch.empty((B, H, M, D), dtype=q.dtype, device=q.device)
-            if ds is None:   # dS not worth keeping for this shape, or no memory for it: recompute it
-                _abi.fa_bwd_dkdv(lib, q, k, v, do, L, delta, dk, dv, causal, sm_scale, dropout, pieces)
-                _abi.fa_bwd_dq(lib, q, k, v, do, L, delta, dq, causal, sm_scale, dropout)
-            elif heads >= B * H:
-                _abi.fa_bwd_dkdv_ds(lib, q, k, v, do, L, delta, dk, dv, ds, causal, sm_scale, dropout, pieces)
-                _abi.fa_bwd_dq_from_ds(lib, k, ds, dq, causal, sm_scale)
-            else:
-                # bounded workspace: one batch entry and `heads` query heads at a time; the dropout
-                # counter of a slice starts where the slice starts in the (B, H, M, N) score tensor
-                for b in range(B):
-                    for h0 in range(0, H, heads):
-                        h1 = min(H, h0 + heads)
-                        hs, ks = slice(h0, h1), slice(h0 // group, -(-h1 // group))
-                        ss = slice(h0 // chunk, h1 // chunk)
-                        bs = slice(b, b + 1)
-                        drop = (dropout[0], dropout[1], dropout[2] + (b * H + h0) * M * N)
-                        _abi.fa_bwd_dkdv_ds(lib, q[bs, hs], k[bs, ks], v[bs, ks], do[bs, hs], L[bs, hs],
-                                            delta[bs, hs], dk[bs, ss], dv[bs, ss], ds, causal, sm_scale, drop, pieces)
-                        _abi.fa_bwd_dq_from_ds(lib, k[bs, ks], ds, dq[bs, hs], causal, sm_scale)
-            if pieces:   # the kernel summed `chunk` heads of every group; add the chunks
-                parts = dk, dv
-                dk, dv = (torch.empty((B, Hk, N, D), dtype=k.dtype, device=q.device) for _ in parts)
-                _abi.fa_sum_slices(lib, parts, (dk, dv))
+            dk_s, dv_s, dq_s = dk, dv, dq
+            if kv_slices > 1:
+                dk_s = _scratch((B, Hk * kv_slices, N, D), torch.float32, q.device)
+                dv_s = None if dk_s is None else _scratch((B, Hk * kv_slices, N, D), torch.float32, q.device)
+                if dv_s is None:     # no memory: whole sums, by as few slices as there are kernels for
+                    if chunk < group and dropout[0] > 0:
+                        raise torch.OutOfMemoryError("flash_attention backward: no memory for the slices of dK and dV")
+                    chunk, kv_pieces, kv_slices, dk_s, dv_s = group, 1, 1, dk, dv
+            if q_pieces > 1:
+                dq_s = _scratch((B, H * q_pieces, M, D), torch.float32, q.device)
+                if dq_s is None:
+                    q_pieces, dq_s = 1, dq
+            kv_code, q_code = kv_pieces if kv_slices > 1 else 0, q_pieces if q_pieces > 1 else 0
+            for b in range(0, B, bn):
+                for h0 in range(0, H, hn):
+                    h1, bs = min(H, h0 + hn), slice(b, b + bn)
+                    hs, ks = slice(h0, h1), slice(h0 // group, h1 // group)      # whole groups of query heads
+                    qt, kt, vt, dot, lt, dt = q[bs, hs], k[bs, ks], v[bs, ks], do[bs, hs], L[bs, hs], delta[bs, hs]
+                    dkt, dvt = (x[bs, ks.start * kv_slices:ks.stop * kv_slices] for x in (dk_s, dv_s))
+                    dqt = dq_s[bs, h0 * q_pieces:h1 * q_pieces]
+                    # the dropout counter of a launch starts where its heads start in the (B, H, M, N) score tensor
+                    drop = (dropout[0], dropout[1], dropout[2] + (b * H + h0) * M * N)
+                    if ds is None:   # dS not worth keeping for this shape, or no memory for it: recompute it
+                        _abi.fa_bwd_dkdv(lib, qt, kt, vt, dot, lt, dt, dkt, dvt, causal, sm_scale, drop, kv_code)
+                        _abi.fa_bwd_dq(lib, qt, kt, vt, dot, lt, dt, dqt, causal, sm_scale, drop, q_code)
+                    else:
+                        _abi.fa_bwd_dkdv_ds(lib, qt, kt, vt, dot, lt, dt, dkt, dvt, ds, causal, sm_scale, drop, kv_code)
+                        _abi.fa_bwd_dq_from_ds(lib, kt, ds, dqt, causal, sm_scale, q_code)
+            sums = ([(dk_s, dk), (dv_s, dv)] if kv_slices > 1 else []) + ([(dq_s, dq)] if q_pieces > 1 else [])
+            if sums:
+                _abi.fa_sum_slices(lib, *zip(*sums))
         return dq, dk, dv, None, None, None, None, None, None
 
 
@@ -308,6 +317,56 @@ def dkdv_heads_per_slice(B, H, group, N, num_cus):
         if group % chunk == 0 and blocks * B * (H // chunk) >= 2 * num_cus:
             return chunk
     return 1
+
+
+# How a backward kernel's workgroups use a compute unit: `slots` of them share it; a step (64 queries or keys) takes one
+# `alone` us, each of a full set `shared` us, and what comes before and behind the steps `around` us.  Measured on long
+# launches (shared) and on launches of less than one workgroup per unit (alone).
+#            slots, alone, shared, around
+_DKDV_128 = (1, 1.7, 2.1, 6.0)
+_DKDV_64 = (2, 1.05, 2.1, 5.0)
+_DQ = (2, 1.1, 1.6, 4.0)
+_DQ_FROM_DS = (2, 1.15, 1.6, 4.0)
+
+
+def _launch_us(pace, tiles, steps, causal, pieces, slice_bytes, num_cus):
+    """Estimated us of a launch of ``tiles`` result tiles of up to ``steps`` steps each, every tile's sum dealt to ``pieces``
+    workgroups.  Under the causal mask workgroups start longest first and average half the longest."""
+    slots, alone, shared, around = pace
+    wgs, per, full = tiles * pieces, steps / pieces, num_cus * slots
+    if causal:
+        t = max(per * alone, tiles * steps / 2 / full * shared)
+    else:
+        rounds = wgs // full
+        rest = wgs - rounds * full
+        t = per * (rounds * shared + (0 if rest == 0 else alone if rest <= num_cus else shared))
+    t += around * max(1.0, wgs / full)
+    # fp32 slices written and read back at 5 TB/s, and the launch that adds them
+    return t if pieces == 1 else t + 3.0 + 2 * wgs * slice_bytes / 5e6
+
+
+def _contraction_pieces(pace, tiles, steps, causal, slice_bytes, num_cus):
+    """Workgroups that share the sum of one result tile (``FA_PIECES``): more than one where a launch is as long as its
+    longest workgroup, or its last round of workgroups is nearly empty, and that costs more than adding the pieces does.
+    A piece keeps at least 8 steps."""
+    best, least = 1, _launch_us(pace, tiles, steps, causal, 1, slice_bytes, num_cus)
+    for n in range(2, 17):
+        if steps < 8 * n:
+            break
+        t = _launch_us(pace, tiles, steps, causal, n, slice_bytes, num_cus)
+        if t < 0.95 * least:
+            best, least = n, t
+    return best
+
+
+def gradient_pieces(B, H, M, N, D, causal, chunk, ds_kept, num_cus):
+    """(pieces of the query axis of a dK/dV tile, pieces of the key axis of a dQ tile).  Counted over all heads, so that
+    launches in turns add up in the same order as one launch.  A workgroup that sums query heads is long as it is."""
+    blocks = lambda n, size: -(-n // size)   # noqa: E731
+    kv = 1 if chunk > 1 else _contraction_pieces(_DKDV_128 if D == 128 else _DKDV_64, blocks(N, 128) * B * H, blocks(M, 64),
+                                                 causal, 2 * 4.0 * 128 * D, num_cus)
+    return kv, _contraction_pieces(_DQ_FROM_DS if ds_kept else _DQ, blocks(M, 128) * B * H, blocks(N, 64), causal,
+                                   4.0 * 128 * D, num_cus)
 
 
 # Largest dS workspace the backward may take (MiB); 0 disables the dS path.  The workspace is
@@ -343,14 +402,19 @@ def even_heads(fit, H, group):
     return -(-(-(-H // launches)) // group) * group
 
 
-def _ds_workspace(lib, device, B, H, M, N, grids=1):
-    """Device memory for dS, or None when the allocator has none left (the caller then recomputes)."""
-    mib = lib.fa_bwd_ds_workspace_mib(B, H, M, N)
-    assert mib > 0
+def _scratch(shape, dtype, device):
+    """Memory that a slower way does without: None when the allocator has none left."""
     try:
-        return torch.empty(grids * (mib << 20), dtype=torch.uint8, device=device)
+        return torch.empty(shape, dtype=dtype, device=device)
     except torch.OutOfMemoryError:
         return None
+
+
+def _ds_workspace(lib, device, B, H, M, N, grids=1):
+    """Device memory for dS, or None (the caller then recomputes)."""
+    mib = lib.fa_bwd_ds_workspace_mib(B, H, M, N)
+    assert mib > 0
+    return _scratch(grids * (mib << 20), torch.uint8, device)
 
 
 def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
