@@ -62,7 +62,7 @@ def test_native_flash_equals_the_python_path(B, H, Hk, M, N, D, causal, layout):
     for a, b in zip(native[:3], python[:3]):
         assert same(a, b)
     assert native[3:] == (None, None)
-    # (the native backward may deal a sum to several workgroups: another order of fp32 additions, one rounding to bf16)
+    # (bound for fp32 sums in another order and one rounding to bf16; test_gradient_pieces.py holds both to the same order)
     for a, b in zip(torch.autograd.grad(native[0], (q, k, v), do), torch.autograd.grad(python[0], (q, k, v), do)):
         assert a.shape == b.shape and a.dtype == b.dtype
         assert (a.float() - b.float()).abs().max() <= 2 ** -7 * b.float().abs().max()
